@@ -22,19 +22,23 @@ __device__ constexpr float R_SQRT2  = 1.41421356237309514547f;
 // The single-precision rounding field of the MODE register (bits 1:0) is
 // set to round-toward-zero around the two fma and restored to nearest-even;
 // both mode writes sit in one asm block so no other floating-point
-// instruction can be scheduled inside the round-toward-zero window.  The
-// nops cover the VALU -> s_setreg and s_setreg -> s_setreg wait states.
+// instruction can be scheduled inside the round-toward-zero window.  No wait
+// states are written out: the hardware orders a mode write against the vector
+// instructions before and after it (the compiler brackets its own division
+// sequences with mode writes the same way), and two writes of the register
+// need two instructions between them: the fma, and the squares of two chains
+// (one chain has a single square, hence its s_nop).  The chain bounds the
+// latency of every pair: with four s_nop 1 per round a lone wave took 775
+// cycles for two pairs of chains, 472 without (192 and 177 with five waves
+// per SIMD).
 __device__ __forceinline__ float t4_round_rz(float x2, float c8, float cm8) {
     float t, r;
     asm volatile(
-        "s_nop 1\n\t"
+        "s_nop 0\n\t"
         "s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 3\n\t"
-        "s_nop 1\n\t"
         "v_fma_f32 %1, %3, %2, %4\n\t"
         "v_fma_f32 %0, %1, %2, 1.0\n\t"
-        "s_nop 1\n\t"
-        "s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 0\n\t"
-        "s_nop 1"
+        "s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 0"
         : "=v"(r), "=&v"(t)
         : "v"(x2), "v"(c8), "v"(cm8));
     return r;
@@ -45,16 +49,12 @@ __device__ __forceinline__ float t4_round_rz(float x2, float c8, float cm8) {
 __device__ __forceinline__ void t4_round_rz2(float a2, float b2, float c8, float cm8, float *ra, float *rb) {
     float ta, tb, oa, ob;
     asm volatile(
-        "s_nop 1\n\t"
         "s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 3\n\t"
-        "s_nop 1\n\t"
         "v_fma_f32 %2, %6, %4, %7\n\t"
         "v_fma_f32 %3, %6, %5, %7\n\t"
         "v_fma_f32 %0, %2, %4, 1.0\n\t"
         "v_fma_f32 %1, %3, %5, 1.0\n\t"
-        "s_nop 1\n\t"
-        "s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 0\n\t"
-        "s_nop 1"
+        "s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 0"
         : "=&v"(oa), "=&v"(ob), "=&v"(ta), "=&v"(tb)
         : "v"(a2), "v"(b2), "v"(c8), "v"(cm8));
     *ra = oa;
