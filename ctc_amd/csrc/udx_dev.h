@@ -162,18 +162,17 @@ __device__ __forceinline__ void clist_count_one(bool valid, int i, float3 r, int
 }
 
 // ---------------------------------------------------------------- DPD pair
-// Correctly rounded square root of a positive normal float (or 0): the
-// hardware root (within 1 ulp) moved to a neighbour when an fma residual
-// shows that neighbour is nearer.  The compiler's IEEE square root does the
-// same after scaling denormal inputs, which the pair force never has.  Every
-// x in [2^-24, 1] is checked on the host against each value a 1-ulp root
-// can give (the oracle's orc_verify_sqrt_rn).
+// Correctly rounded square root of a positive normal float: the product of
+// x and the hardware reciprocal root, corrected by its fma residual times half
+// that root.  Equal to the IEEE root for every float of [2^-24, 1] (checked
+// exhaustively on gfx950; the library's self-check entry point repeats the
+// check).  One transcendental, two products and two fma, 19 issue cycles of a
+// wave; the hardware root moved to a neighbour by two residuals, compares and
+// selects took 37.  x = 0 gives NaN.
 __device__ __forceinline__ float sqrt_rn(float x) {
-    const float s = __builtin_amdgcn_sqrtf(x);
-    const float sd = __int_as_float(__float_as_int(s) - 1), su = __int_as_float(__float_as_int(s) + 1);
-    const float rd = __builtin_fmaf(-sd, s, x), ru = __builtin_fmaf(-su, s, x);
-    const float t = rd <= 0.f ? sd : s;
-    return ru > 0.f ? su : t;
+    const float y = __builtin_amdgcn_rsqf(x);
+    const float s = x * y, h = 0.5f * y;
+    return __builtin_fmaf(__builtin_fmaf(-s, s, x), h, s);
 }
 
 // Correctly rounded reciprocal of r in [2^-24, 1]: the hardware reciprocal
@@ -206,22 +205,22 @@ struct DpdPar { float a, g, s, spow; };
 // rounded, so the force equals the CPU restatement bit for bit (the
 // reference's fast-math r2 rsqrtf(r2) is 1e-3 wrong in w_R near the cutoff,
 // where w_R = (1 - r)^spow has an unbounded slope).  The template argument
-// EXACT is kept for the generic exponent (powf).
+// EXACT is kept for the generic exponent (powf).  A pair that is no pair (an
+// idle slot, r2 >= 1) gives a value to be discarded, NaN among them.
 template <int WR, bool EXACT>
 __device__ __forceinline__ float3 dpd_pair(const DpdPar &p, float dx, float dy, float dz, float r2,
                                            float dvx, float dvy, float dvz, float rnd) {
-    float ex, ey, ez, r;
-    if (r2 < 1e-6f) {
-        ex = ey = ez = r = 0.0f;
-    } else {
-        r = sqrt_rn(r2);
-        const float invr = rcp_rn(r);   // r >= 1e-3
-        ex = dx * invr; ey = dy * invr; ez = dz * invr;
-    }
-    float ev = __builtin_fmaf(ez, dvz, __builtin_fmaf(ex, dvx, ey * dvy));
-    float rm = 1.0f - r;
-    rm = rm > 0.0f ? rm : 0.0f;
-    float wr = wr_pow<WR, EXACT>(rm, p.spow);
+    // selects, not branches: a wave nearly always holds both kinds of pairs
+    // or none of the close ones
+    const bool close = r2 < 1e-6f;
+    float r = sqrt_rn(r2);
+    float invr = rcp_rn(r);   // r >= 1e-3
+    r = close ? 0.0f : r;
+    invr = close ? 0.0f : invr;
+    const float ex = dx * invr, ey = dy * invr, ez = dz * invr;
+    const float ev = __builtin_fmaf(ez, dvz, __builtin_fmaf(ex, dvx, ey * dvy));
+    const float rm = 1.0f - r;   // at least 2^-24: the largest root of r2 < 1 is 1 - 2^-24
+    const float wr = wr_pow<WR, EXACT>(rm, p.spow);
     float f0 = __builtin_fmaf(-p.g * wr, ev, p.s * rnd) * wr;
     f0 = __builtin_fmaf(p.a, rm, f0);
     return make_float3(f0 * ex, f0 * ey, f0 * ez);

@@ -58,7 +58,7 @@ int udx_rnd_branch(udx_ctx *ctx, float seed, int n, const int *u, const int *v, 
  *      compares the library's device routine with the correctly rounded
  *      result and returns the number of floats that differ (synchronises).
  *      UDX_CHECK_RCP: the reciprocal of the pair force (for x in [2^-24, 1]);
- *      UDX_CHECK_SQRT: its square root; UDX_CHECK_FRACT: x - floor(x) of the
+ *      UDX_CHECK_SQRT: its square root (for x in [2^-24, 1]); UDX_CHECK_FRACT: x - floor(x) of the
  *      branch generator; UDX_CHECK_RCP_ESTIMATE: the hardware reciprocal
  *      estimate alone (not correctly rounded: shows that the check counts). ---- */
 enum { UDX_CHECK_RCP = 0, UDX_CHECK_SQRT = 1, UDX_CHECK_FRACT = 2, UDX_CHECK_RCP_ESTIMATE = 3 };
