@@ -352,7 +352,7 @@ int udx_fluforces_ini(udx_ctx *ctx, int Lx, int Ly, int Lz, int maxp, udx_flufor
     f->maxp = maxp;
     f->trunks.ini();
     int s = UDX_OK;
-    if (!s) s = dev_alloc(&f->pos, maxp);
+    if (!s) s = dev_alloc(&f->pos, (size_t)maxp + POS_PAD);
     if (!s) s = dev_alloc(&f->vel, maxp);
     if (!s) s = dev_alloc(&f->seeds_dev, 27);
     if (!s) s = dev_alloc(&f->pairs_dev, 1);
@@ -520,7 +520,7 @@ int udx_flu_ini(udx_ctx *ctx, const udx_flu_conf *conf, udx_flu **out) {
     f->seed_cap = 0;
     int s = UDX_OK;
     for (int b = 0; b < 2 && !s; b++) {
-        s = dev_alloc(&f->pos[b], conf->maxp);
+        s = dev_alloc(&f->pos[b], (size_t)conf->maxp + POS_PAD);
         if (!s) s = dev_alloc(&f->vel[b], conf->maxp);
     }
     if (!s) s = dev_alloc(&f->ff, conf->maxp);

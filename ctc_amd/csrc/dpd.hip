@@ -288,6 +288,75 @@ using PassTag = std::integral_constant<bool, B>;
 // the order of the additions is that of one pass)
 enum { PH_ALL = 0, PH_BULK = 1, PH_HALO = 2 };
 
+// stress 1/2 f_a dr_b of a particle's pairs (src/pair/dev.h:87-100)
+struct Stress {
+    float xx, xy, xz, yy, yz, zz;
+};
+
+// What becomes of a particle's sums (called by every lane of a wave; mine: the
+// lane has a particle i to finish): the force stored or added and, where the
+// move is fused, the step's total force (the wall sum added for the particles
+// near a wall: 0 + sum, then + wall, as ff = sum and ff += wall), the
+// kick-drift, the bounce-back and the wrap of move_f4_wall, then the count
+// into the next step's x slabs (MOVE: the single-box kernels; A.opos without
+// MOVE: a batch without walls, where a particle listed for the halo launch is
+// moved there).
+template <int MOVE, bool STRESS>
+__device__ __forceinline__ void finish(const DpdK &A, const DpdP &P, bool mine, int i, const float4 &pi,
+                                       const float4 &vi, float3 f, bool wnear, float3 ws, const Stress &st) {
+    if (MOVE || A.opos) {
+        float4 p = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (mine) {
+            UDX_GLOBAL f4v *f4 = (UDX_GLOBAL f4v *)A.ff + i;
+            float gx = 0.f + f.x, gy = 0.f + f.y, gz = 0.f + f.z;
+            if (MOVE == 2 && wnear) {
+                gx = gx + ws.x;
+                gy = gy + ws.y;
+                gz = gz + ws.z;
+            }
+            *f4 = f4v{gx, gy, gz, 0.f};
+            p = pi;
+            float4 v = vi;
+            kick_drift(A.mdt, A.mmass, A.max_, gx, &p.x, &v.x);
+            kick_drift(A.mdt, A.mmass, A.may, gy, &p.y, &v.y);
+            kick_drift(A.mdt, A.mmass, A.maz, gz, &p.z, &v.z);
+            if (MOVE == 2) {
+                float r[3] = {p.x, p.y, p.z}, u[3] = {v.x, v.y, v.z};
+                if (sdf_bounce(A.sdf, A.wv, A.mdt, r, u)) {
+                    p.x = r[0]; p.y = r[1]; p.z = r[2];
+                    v.x = u[0]; v.y = u[1]; v.z = u[2];
+                }
+            }
+            p.x = wrap_coord(p.x, (float)P.Lx);
+            p.y = wrap_coord(p.y, (float)P.Ly);
+            p.z = wrap_coord(p.z, (float)P.Lz);
+            *((UDX_GLOBAL f4v *)A.opos + i) = f4v{p.x, p.y, p.z, 0.f};
+            *((UDX_GLOBAL f4v *)A.ovel + i) = f4v{v.x, v.y, v.z, 0.f};
+        }
+        clist_count_one(mine, i, make_float3(p.x, p.y, p.z), A.sc.L[0], A.sc.L[1], A.sc.L[2], A.sc.sub,
+                        A.sc.counts, A.sc.cellslot, A.sc.slab0);
+    } else if (mine) {
+        if (A.ff_stride == 4) {
+            UDX_GLOBAL f4v *f4 = (UDX_GLOBAL f4v *)A.ff + i;
+            f4v o = {0.f, 0.f, 0.f, 0.f};
+            if (A.accumulate) o = *f4;
+            *f4 = f4v{o.x + f.x, o.y + f.y, o.z + f.z, 0.f};
+        } else {
+            UDX_GLOBAL float *f3 = gptr(A.ff) + 3 * (long)i;
+            if (A.accumulate) {
+                f3[0] += f.x; f3[1] += f.y; f3[2] += f.z;
+            } else {
+                f3[0] = f.x; f3[1] = f.y; f3[2] = f.z;
+            }
+        }
+        if (STRESS) {
+            UDX_GLOBAL float *s6 = gptr(A.ss) + 6 * (long)i;
+            s6[0] += st.xx; s6[1] += st.xy; s6[2] += st.xz;
+            s6[3] += st.yy; s6[4] += st.yz; s6[5] += st.zz;
+        }
+    }
+}
+
 // The force pass of one block of NT consecutive particles starting at i
 // = first + threadIdx.x; QC (a power of two) queued pairs per lane.
 //
@@ -753,64 +822,8 @@ __device__ __forceinline__ void dpd_block(const DpdK &A, int first) {
         }
     }
 
-    if (MOVE || A.opos) {
-        // the step's total force (the wall sum added for the particles near a
-        // wall: 0 + sum, then + wall, as ff = sum and ff += wall), the
-        // kick-drift, the bounce-back and the wrap of move_f4_wall, then the
-        // count into the next step's x slabs (MOVE: the single-box kernel;
-        // A.opos without MOVE: a batch without walls, where a particle
-        // listed for the halo launch is moved there)
-        const bool mine = active && !listed;
-        float4 p = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (mine) {
-            UDX_GLOBAL f4v *f4 = (UDX_GLOBAL f4v *)A.ff + i;
-            float gx = 0.f + fx, gy = 0.f + fy, gz = 0.f + fz;
-            if (MOVE == 2 && wnear) {
-                gx = gx + wsx;
-                gy = gy + wsy;
-                gz = gz + wsz;
-            }
-            *f4 = f4v{gx, gy, gz, 0.f};
-            p = pi;
-            float4 v = vi;
-            kick_drift(A.mdt, A.mmass, A.max_, gx, &p.x, &v.x);
-            kick_drift(A.mdt, A.mmass, A.may, gy, &p.y, &v.y);
-            kick_drift(A.mdt, A.mmass, A.maz, gz, &p.z, &v.z);
-            if (MOVE == 2) {
-                float r[3] = {p.x, p.y, p.z}, u[3] = {v.x, v.y, v.z};
-                if (sdf_bounce(A.sdf, A.wv, A.mdt, r, u)) {
-                    p.x = r[0]; p.y = r[1]; p.z = r[2];
-                    v.x = u[0]; v.y = u[1]; v.z = u[2];
-                }
-            }
-            p.x = wrap_coord(p.x, (float)Lx);
-            p.y = wrap_coord(p.y, (float)Ly);
-            p.z = wrap_coord(p.z, (float)Lz);
-            *((UDX_GLOBAL f4v *)A.opos + i) = f4v{p.x, p.y, p.z, 0.f};
-            *((UDX_GLOBAL f4v *)A.ovel + i) = f4v{v.x, v.y, v.z, 0.f};
-        }
-        clist_count_one(mine, i, make_float3(p.x, p.y, p.z), A.sc.L[0], A.sc.L[1], A.sc.L[2], A.sc.sub,
-                        A.sc.counts, A.sc.cellslot, A.sc.slab0);
-    } else if (active && !listed) {
-        if (A.ff_stride == 4) {
-            UDX_GLOBAL f4v *f4 = (UDX_GLOBAL f4v *)A.ff + i;
-            f4v o = {0.f, 0.f, 0.f, 0.f};
-            if (A.accumulate) o = *f4;
-            *f4 = f4v{o.x + fx, o.y + fy, o.z + fz, 0.f};
-        } else {
-            UDX_GLOBAL float *f3 = gptr(A.ff) + 3 * (long)i;
-            if (A.accumulate) {
-                f3[0] += fx; f3[1] += fy; f3[2] += fz;
-            } else {
-                f3[0] = fx; f3[1] = fy; f3[2] = fz;
-            }
-        }
-        if (STRESS) {
-            UDX_GLOBAL float *s6 = gptr(A.ss) + 6 * (long)i;
-            s6[0] += sxx; s6[1] += sxy; s6[2] += sxz;
-            s6[3] += syy; s6[4] += syz; s6[5] += szz;
-        }
-    }
+    finish<MOVE, STRESS>(A, P, active && !listed, i, pi, vi, make_float3(fx, fy, fz), wnear,
+                         make_float3(wsx, wsy, wsz), Stress{sxx, sxy, sxz, syy, syz, szz});
     if (A.pairs) {
         unsigned long long c = (unsigned long long)npair;
 #pragma unroll
@@ -864,6 +877,515 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(5))) void k_
     }
     const DpdK &A = boxes[lo];
     dpd_block<WR, EXACT, NT, QC, SCAP_BATCH, false, PHASE>(A, A.i0 + (blk - bblock[lo]) * NT);
+}
+
+// ---------------------------------------------------------------- one block per 64 particles
+// The same sums with a whole block per 64 particles, for boxes with too few
+// particles to fill the chip with k_dpd.  There a lane owns a particle from its
+// first candidate to its last pair, a serial chain of about 130 thousand
+// cycles, and a small box is one such chain long however many lanes are idle.
+// Here nine waves share 64 consecutive particles (the home particles, one per
+// lane in every wave) in three steps:
+//  - candidates: wave (dz, dy) tests the candidates of that row against the
+//    lanes' home particles; the hits are bits of a mask per lane;
+//  - pairs: the hits of all home particles form one list, by home particle
+//    and, inside, in the order of the sums (counts per home and row, a scan);
+//    every lane of the block evaluates pairs of that list, whoever's they
+//    are, and leaves the force in the pair's slot in LDS;
+//  - sums: a lane per home particle and component adds its slots in order,
+//    then the particle is finished (the additions of k_dpd one for one, so the
+//    forces are the same bits).
+// A list longer than the LDS slots is worked off in windows; a run of more
+// than 64 candidates for some lane makes the block go run by run, 64 at a time.
+// What bounds it is the latency of its eight dependent steps (global loads of
+// the particle, the slab starts, the candidates, the pairs' particles and the
+// slot atomic of the next count, and the barriers between them), about 20
+// thousand cycles a block.  Measured per launch, k_dpd against this: 12288
+// particles (16^3, density 3) 56.5 -> 12.5 us; 63240 (31x17x24, density 5) 76
+// -> 34 us.  With many blocks per CU the barriers cost more than the idle
+// lanes of k_dpd (48^3, density 10: 431 -> 590 us): dpd_small() has the line.
+constexpr int CO_WAVES = 9, CO_THREADS = 64 * CO_WAVES;
+constexpr int CO_STAGE = 128;               // candidates a wave stages in LDS
+constexpr int CO_CAP = 3072;                // pair slots of a block (density 10 has about 2600)
+constexpr unsigned CO_DENSE = 0xFFu;        // a row with more than 64 candidates in a run
+
+// v summed over the lanes up to this one
+__device__ __forceinline__ int wave_scan_add(int v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);   // row_shr:1
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);   // row_bcast:15
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);   // row_bcast:31
+    return v;
+}
+
+// x, y, z of particle j + K, K a constant folded into the load
+__device__ __forceinline__ f3v pos_at(const UDX_GLOBAL f4v *p, unsigned byte, int k) {
+    return *(const UDX_GLOBAL f3v *)((const UDX_GLOBAL char *)p + (size_t)byte + 16 * k);
+}
+
+// hits of up to 64 candidates as bits, candidate k at bit 31 - (k mod 32) of
+// word k / 32: the sign of r2 - 1, shifted in from the right.  at(k) reads the
+// lane's candidate k, for k up to seven past the last one.
+struct Mask64 {
+    unsigned w[2];
+};
+template <class At>
+__device__ __forceinline__ Mask64 test64(int n, float ax, float ay, float az, At at) {
+    Mask64 m{{0u, 0u}};
+#pragma unroll
+    for (int c = 0; c < 2; c++) {
+        if (!wave_any(n > 32 * c)) break;
+        unsigned b = 0;
+        int sh = 32;
+        f3v q[4], nx[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) q[u] = at(32 * c + u);
+#pragma unroll
+        for (int g = 0; g < 8; g++) {
+            if (g && !wave_any(n > 32 * c + 4 * g)) break;
+            if (g < 7)
+#pragma unroll
+                for (int u = 0; u < 4; u++) nx[u] = at(32 * c + 4 * (g + 1) + u);
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                const float dx = ax - q[u].x, dy = ay - q[u].y, dz = az - q[u].z;
+                const float r2 = __builtin_fmaf(dz, dz, __builtin_fmaf(dx, dx, dy * dy));
+                b = __builtin_amdgcn_alignbit(b, __float_as_uint(r2 - 1.0f), 31);
+            }
+            sh -= 4;
+#pragma unroll
+            for (int u = 0; u < 4; u++) q[u] = nx[u];
+        }
+        b <<= sh & 31;
+        const int left = n - 32 * c;
+        m.w[c] = left >= 32 ? b : (left > 0 ? b & ~(0xFFFFFFFFu >> left) : 0u);
+    }
+    return m;
+}
+
+// smallest and largest value over the wave's lanes
+__device__ __forceinline__ int wave_min(int v) {
+    v = min(v, __builtin_amdgcn_update_dpp(0x7fffffff, v, 0x111, 0xf, 0xf, false));
+    v = min(v, __builtin_amdgcn_update_dpp(0x7fffffff, v, 0x112, 0xf, 0xf, false));
+    v = min(v, __builtin_amdgcn_update_dpp(0x7fffffff, v, 0x114, 0xf, 0xf, false));
+    v = min(v, __builtin_amdgcn_update_dpp(0x7fffffff, v, 0x118, 0xf, 0xf, false));
+    v = min(v, __builtin_amdgcn_update_dpp(0x7fffffff, v, 0x142, 0xa, 0xf, false));
+    v = min(v, __builtin_amdgcn_update_dpp(0x7fffffff, v, 0x143, 0xc, 0xf, false));
+    return __builtin_amdgcn_readlane(v, 63);
+}
+__device__ __forceinline__ int wave_max(int v) { return -wave_min(-v); }
+
+struct CoopLds {
+    float4 hp[64], hv[64];
+    union {
+        float4 stage[CO_WAVES][CO_STAGE + 8];   // a wave's candidates while it tests them
+        // the list: a pair's home | wrap << 8, its other particle and, across
+        // the boundary, its noise indices; then the three force components
+        unsigned item[4][CO_CAP];
+    };
+    float sum[2][3][64];       // the home particles' solvent and wall sums
+    unsigned cnt[64][5];       // counts of the home particle's rows, a byte each (bulk rows, wrapped rows)
+};
+
+// candidates of one run of cells for a lane: j .. j + n - 1, the periodic wrap
+// wx of the run's cells seen from the home particle, and the home particle's x
+// in the run's frame; for a wrapped run the noise indices: the home particle's
+// position in the packed list of fragment w, and what a candidate's index in
+// the opposite fragment's list exceeds its particle index by
+struct Run {
+    int j, n, wx, x0, x1, aid, bb;
+    float ax;
+    bool on;
+};
+
+template <int WR, int MOVE>
+__device__ __forceinline__ void coop_block(const DpdK &A, int first, CoopLds &S) {
+    const int tid = threadIdx.x, lane = tid & 63, row = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const DpdP P = dpd_view(A);
+    const int Lx = P.Lx, Ly = P.Ly, Lz = P.Lz, i0 = P.i0;
+    const UDX_GLOBAL f4v *const pos = P.pos + i0, *const vel = P.vel + i0;
+    const int i = first - i0 + lane;   // of the box, as every particle index below
+    // (loads ahead of the particle count: the arrays hold nmax particles)
+    float4 pi = make_float4(0.f, 0.f, 0.f, 0.f), vi = pi;
+    if (i < P.nmax) {
+        pi = P.p(i + i0);
+        if (row == 0) vi = P.v(i + i0);
+    }
+    const bool active = i < P.nmax && i + i0 < P.starts[Lx * Ly * Lz];
+    int cx = 0, cy = 0, cz = 0;
+    float rx = 0.f, ry = 0.f, rz = 0.f;   // position inside the cell
+    if (active) {
+        cell_coord(pi.x, Lx, &cx);
+        cell_coord(pi.y, Ly, &cy);
+        cell_coord(pi.z, Lz, &cz);
+        rx = (float)((double)pi.x + 0.5 * (double)Lx - (double)cx);
+        ry = (float)((double)pi.y + 0.5 * (double)Ly - (double)cy);
+        rz = (float)((double)pi.z + 0.5 * (double)Lz - (double)cz);
+    }
+    if (row == 0) {
+        S.hp[lane] = pi;
+        S.hv[lane] = vi;
+    }
+    const bool edge =
+        active && P.periodic && (cx == 0 || cx == Lx - 1 || cy == 0 || cy == Ly - 1 || cz == 0 || cz == Lz - 1);
+    const bool edges = wave_any(edge);   // the same in every wave
+    const bool wnear = MOVE == 2 && active && !sdf_far(A.sdf, pi.x, pi.y, pi.z);
+    const int dz = row / 3 - 1, dy = row % 3 - 1;   // this wave's row of cells
+    float acc[2] = {0.f, 0.f};   // component `row` of the home particle's solvent and wall sums (waves 0-2)
+
+    // One list of pairs from start to sums.  r1, r2: the lane's runs of this
+    // wave's row, r1 before r2 in the order of the sums; wrapped1: r1 lies
+    // across the periodic boundary (r2 always does), and wrapped rows come
+    // after all the others.  load(p) and its chains evaluate slot p.
+    auto pass = [&](auto wall, const Run &r1, const Run &r2, bool second, bool wrapped1, int wy, int wz,
+                    const UDX_GLOBAL f4v *cand, auto in_of) {
+        constexpr bool WALL = decltype(wall)::value;
+        const bool wraps = !WALL && edges;
+        const float ay = pi.y - (float)(wy * Ly), az = pi.z - (float)(wz * Lz);
+        // the lanes are consecutive particles: the union of their runs is one
+        // range (two with r2), staged in LDS with coalesced loads where it fits
+        // (one round trip; per-lane loads of the candidates are bound by the
+        // address unit)
+        const int lo1 = wave_min(r1.n > 0 ? r1.j : 0x7fffffff), hi1 = wave_max(r1.n > 0 ? r1.j + r1.n : 0);
+        int lo2 = 0, hi2 = 0;
+        if (second) {
+            lo2 = wave_min(r2.n > 0 ? r2.j : 0x7fffffff);
+            hi2 = wave_max(r2.n > 0 ? r2.j + r2.n : 0);
+        }
+        const int len1 = max(hi1 - lo1, 0), len = len1 + max(hi2 - lo2, 0);
+        const bool staged = !WALL && len <= CO_STAGE;
+        unsigned char *const cnt = (unsigned char *)S.cnt[lane];
+        unsigned long long npair = 0;
+        // sel < 0: every run, its first 64 candidates; else one run (the rows'
+        // unwrapped runs, then the wrapped rows' first and second runs),
+        // candidates from `skip`
+        int sel = -1, skip = 0;
+        for (;;) {
+            const bool on1 = sel < 0 || (sel < 9 ? sel == row && !wrapped1 : sel == 9 + 2 * row && wrapped1);
+            const bool on2 = sel < 0 || sel == 10 + 2 * row;
+            const int n1 = on1 ? r1.n - skip : 0, n2 = second && on2 ? r2.n - skip : 0;
+            Mask64 m1{{0u, 0u}}, m2{{0u, 0u}};
+            if (staged) {
+                float4 *const st = S.stage[row];
+                __builtin_amdgcn_wave_barrier();
+                f3v x[CO_STAGE / 64];
+#pragma unroll
+                for (int t = 0; t < CO_STAGE / 64; t++)
+                    if (len > 64 * t) {
+                        const int k = min(64 * t + lane, len - 1);
+                        x[t] = pos_at(cand, (unsigned)(k < len1 ? lo1 + k : lo2 + k - len1) * 16u, 0);
+                    }
+#pragma unroll
+                for (int t = 0; t < CO_STAGE / 64; t++)
+                    if (len > 64 * t) st[64 * t + lane] = make_float4(x[t].x, x[t].y, x[t].z, 0.f);
+                __builtin_amdgcn_wave_barrier();
+                const int o1 = n1 > 0 ? r1.j + skip - lo1 : 0, o2 = n2 > 0 ? len1 + r2.j + skip - lo2 : 0;
+                m1 = test64(n1, r1.ax, ay, az, [&](int k) { return *(const f3v *)&st[o1 + k]; });
+                if (second) m2 = test64(n2, r2.ax, ay, az, [&](int k) { return *(const f3v *)&st[o2 + k]; });
+            } else {
+                const unsigned b1 = (unsigned)(n1 > 0 ? r1.j + skip : 0) * 16u;
+                m1 = test64(n1, r1.ax, ay, az, [&](int k) { return pos_at(cand, b1, k); });
+                if (second) {
+                    const unsigned b2 = (unsigned)(n2 > 0 ? r2.j + skip : 0) * 16u;
+                    m2 = test64(n2, r2.ax, ay, az, [&](int k) { return pos_at(cand, b2, k); });
+                }
+            }
+            if (!WALL && row == 4 && !wrapped1) {
+                // the home particle itself
+                const int k = i - r1.j - skip;
+                if (k >= 0 && k < 32) m1.w[0] &= ~(0x80000000u >> k);
+                if (k >= 32 && k < 64) m1.w[1] &= ~(0x80000000u >> (k - 32));
+            }
+            const unsigned c1 = (unsigned)(__popc(m1.w[0]) + __popc(m1.w[1]));
+            const unsigned c2 = second ? (unsigned)(__popc(m2.w[0]) + __popc(m2.w[1])) : 0u;
+            const unsigned cb = wrapped1 ? 0u : c1, cw = (wrapped1 ? c1 : 0u) + c2;
+            cnt[row] = (unsigned char)(!wrapped1 && n1 > 64 ? CO_DENSE : cb);
+            if (wraps) cnt[9 + row] = (unsigned char)((wrapped1 && n1 > 64) || n2 > 64 ? CO_DENSE : cw);
+            __syncthreads();
+
+            // where each run of the home particles goes in the list
+            unsigned word[5];
+            auto counts = [&]() {
+#pragma unroll
+                for (int k = 0; k < 5; k++) word[k] = k < 3 || wraps ? S.cnt[lane][k] : 0u;
+                if (wraps) word[4] &= 0xFFFFu;
+                else word[2] &= 0xFFu;
+            };
+            counts();
+            unsigned dn = 0;
+#pragma unroll
+            for (int k = 0; k < 5; k++) dn |= word[k] & (word[k] >> 7) & 0x01010101u;
+            const bool dense = wave_any(dn != 0u);   // the same in every wave
+            if (dense) {
+                __syncthreads();
+                if (sel < 0) {
+                    sel = 0;
+                    continue;
+                }
+                cnt[row] = (unsigned char)cb;
+                if (wraps) cnt[9 + row] = (unsigned char)cw;
+                __syncthreads();
+                counts();
+            }
+            int tot = 0;
+#pragma unroll
+            for (int k = 0; k < 5; k++) tot = (int)__builtin_amdgcn_sad_u8(word[k], 0u, (unsigned)tot);
+            const int end = wave_scan_add(tot), off = end - tot;
+            const int T = __builtin_amdgcn_readlane(end, 63);
+            npair += (unsigned long long)T;
+            // entries of the list before slot `slot` of this lane's home particle
+            auto before = [&](int slot) {
+                unsigned p = (unsigned)off;
+#pragma unroll
+                for (int k = 0; k < 5; k++) {
+                    const int b = slot - 4 * k;
+                    const unsigned keep = b <= 0 ? 0u : (b >= 4 ? 0xFFFFFFFFu : (1u << (8 * b)) - 1u);
+                    p = __builtin_amdgcn_sad_u8(word[k] & keep, 0u, p);
+                }
+                return (int)p;
+            };
+            int at1 = before(row), at2 = 0;
+            if (wraps) {
+                at2 = before(9 + row);
+                if (wrapped1) {
+                    at1 = at2;
+                    at2 += (int)c1;
+                }
+            }
+
+            for (int c0 = 0; c0 < T; c0 += CO_CAP) {
+                if (c0) __syncthreads();
+                // the hits of the window into their slots
+                auto put = [&](const Mask64 &mm, const Run &r, int at, bool wrapped) {
+                    const unsigned wc = wrapped ? wcode(r.wx, wy, wz) : W_NONE, meta = (unsigned)lane | wc << 8;
+                    const bool home_first = frag_d2i(r.wx, wy, wz) < frag_d2i(-r.wx, -wy, -wz);
+#pragma unroll
+                    for (int c = 0; c < 2; c++) {
+                        unsigned b = mm.w[c];
+                        while (wave_any(b != 0u)) {
+                            const int k = __builtin_clz(b | 1u);
+                            const int p = at - c0, jj = r.j + skip + 32 * c + k;
+                            if (b && p >= 0 && p < CO_CAP) {
+                                S.item[0][p] = meta;
+                                S.item[1][p] = (unsigned)jj;
+                                if (!WALL && wrapped) {
+                                    S.item[2][p] = (unsigned)(home_first ? r.aid : r.bb + jj);
+                                    S.item[3][p] = (unsigned)(home_first ? r.bb + jj : r.aid);
+                                }
+                            }
+                            at += b ? 1 : 0;
+                            b &= ~(0x80000000u >> k);
+                        }
+                    }
+                };
+                put(m1, r1, at1, wrapped1);
+                if (second) put(m2, r2, at2, true);
+                __syncthreads();
+
+                // the window's pairs over all lanes, two per lane and turn.  A
+                // lane past the list evaluates its block's first particle
+                // against candidate 0 (never slot values: another lane's force
+                // may be in them by now)
+                const int Tw = min(T - c0, CO_CAP);
+                auto load = [&](int p) {
+                    const bool ok = p < Tw;
+                    const int k = ok ? p : 0;
+                    return in_of(k, ok ? S.item[0][k] : W_NONE << 8, ok ? (int)S.item[1][k] : 0);
+                };
+                auto store = [&](int p, const PairIn &a, float x) {
+                    const float3 f =
+                        dpd_pair<WR, false>(P.par, a.dx, a.dy, a.dz, a.r2, a.dvx, a.dvy, a.dvz, x * R_SQRT2);
+                    if (p < Tw) {
+                        S.item[0][p] = __float_as_uint(f.x);
+                        S.item[1][p] = __float_as_uint(f.y);
+                        S.item[2][p] = __float_as_uint(f.z);
+                    }
+                };
+                int p = tid;
+                for (; wave_any(p + CO_THREADS < Tw); p += 2 * CO_THREADS) {
+                    const PairIn a = load(p), b = load(p + CO_THREADS);
+                    float xa = a.x, xb = b.x;
+                    logistic18x2(&xa, &xb);
+                    store(p, a, xa);
+                    store(p + CO_THREADS, b, xb);
+                }
+                if (wave_any(p < Tw)) {
+                    const PairIn a = load(p);
+                    store(p, a, logistic18(a.x));
+                }
+                __syncthreads();
+
+                // the sums, in order: a wave per component, eight slots in flight
+                if (row < 3) {
+                    const int ea = max(off, c0) - c0, ee = min(end, c0 + CO_CAP) - c0;
+                    const unsigned *const it = S.item[row];
+                    unsigned f[8], g[8];
+#pragma unroll
+                    for (int u = 0; u < 8; u++) f[u] = it[ea + u < ee ? ea + u : 0];
+                    for (int k = ea; wave_any(k < ee); k += 8) {
+#pragma unroll
+                        for (int u = 0; u < 8; u++) g[u] = it[k + 8 + u < ee ? k + 8 + u : 0];
+#pragma unroll
+                        for (int u = 0; u < 8; u++) {
+                            if (k + u < ee) acc[WALL ? 1 : 0] += __uint_as_float(f[u]);
+                            f[u] = g[u];
+                        }
+                    }
+                }
+            }
+            if (sel < 0) break;
+            if (dense) {
+                skip += 64;
+            } else {
+                sel++;
+                skip = 0;
+                if (sel == (wraps ? 27 : 9)) break;
+            }
+            __syncthreads();
+        }
+        unsigned long long *const count = WALL ? A.wpairs : A.pairs;
+        if (count && tid == 0 && npair) atomicAdd(count, npair);
+    };
+
+    // ---- solvent pairs.  r1: the part of the row inside the box, or, where
+    // the row lies across the y or z boundary, the wrapped run of smaller dx;
+    // r2: the run across the x boundary, or the second wrapped run
+    {
+        int yy = cy + dy, zz = cz + dz;
+        const int wy = yy < 0 ? -1 : (yy >= Ly ? 1 : 0), wz = zz < 0 ? -1 : (zz >= Lz ? 1 : 0);
+        const bool yz = (wy | wz) != 0;
+        yy -= wy * Ly;
+        zz -= wz * Lz;
+        const float hw = row_halfwidth(dy, dz, ry, rz);
+        const bool reach = active && hw >= 0.f;
+        const int base = Lx * (yy + Ly * zz);
+        Run r1{0, 0, 0, cx > 0 ? cx - 1 : 0, cx + 1 < Lx ? cx + 1 : Lx - 1, 0, 0, pi.x, reach && !yz};
+        Run r2 = r1;
+        r2.on = false;
+        if (edge && reach) {
+            if (yz) {
+                r1.on = xrun(0, cx, Lx, &r1.x0, &r1.x1, &r1.wx);
+                r2.on = xrun(1, cx, Lx, &r2.x0, &r2.x1, &r2.wx);
+            } else {
+                r2.on = (xrun(0, cx, Lx, &r2.x0, &r2.x1, &r2.wx) && r2.wx != 0) ||
+                        (xrun(1, cx, Lx, &r2.x0, &r2.x1, &r2.wx) && r2.wx != 0);
+            }
+        }
+        // candidates of the run's cells within reach along x: cut to x slabs where the list has them
+        auto range = [&](Run &r) {
+            r.ax = pi.x - (float)(r.wx * Lx);
+            int lo, hi;
+            const UDX_GLOBAL int *st = P.bstarts;
+            if (!st) {
+                st = P.starts;
+                lo = base + r.x0;
+                hi = base + r.x1;
+            } else {
+                const int c = (cx - r.wx * Lx) * P.sub;
+                lo = c + (int)__builtin_floorf((rx - hw) * (float)P.sub);
+                hi = c + (int)__builtin_floorf((rx + hw) * (float)P.sub);
+                lo = max(lo, r.x0 * P.sub);
+                hi = min(hi, r.x1 * P.sub + P.sub - 1);
+                r.on = r.on && lo <= hi;
+                lo += base * P.sub;
+                hi += base * P.sub;
+            }
+            const int a = st[r.on ? lo : 0], e = st[r.on ? hi + 1 : 0];
+            r.n = e - a;
+            r.j = r.n > 0 ? a - i0 : 0;
+        };
+        auto lists = [&](Run &r) {
+            const int fid = frag_d2i(r.wx, wy, wz), anti = frag_d2i(-r.wx, -wy, -wz);
+            const int fo = A.foff[fid], ao = A.foff[anti];
+            const int hs = P.starts[cx + Lx * (cy + Ly * cz)] - i0;
+            r.aid = P.fss[fo + frag_cell(r.wx, wy, wz, cx, cy, cz, Lx, Ly)] - P.fss[fo] + (i - hs);
+            r.bb = P.fss[ao + frag_cell(-r.wx, -wy, -wz, r.x0, yy, zz, Lx, Ly)] - P.fss[ao] -
+                   (P.starts[r.x0 + base] - i0);
+        };
+        range(r1);
+        const bool second = edges && wave_any(r2.on);
+        if (second) range(r2);
+        if (edges) {
+            if (r1.on && yz) lists(r1);
+            if (r2.on) lists(r2);
+        }
+        pass(PassTag<false>{}, r1, r2, second, yz, wy, wz, pos, [&](int k, unsigned meta, int j) {
+            const unsigned home = meta & 63u, wc = meta >> 8;
+            const int ih = first - i0 + (int)home;
+            const float4 h = S.hp[home], hv = S.hv[home];
+            const f3v pj = pos_at(pos, (unsigned)j * 16u, 0), vj = pos_at(vel, (unsigned)j * 16u, 0);
+            unsigned u = (unsigned)max(ih, j), v = (unsigned)min(ih, j);
+            float ax = h.x, hy = h.y, hz = h.z, seed = P.seeds[26];
+            if (edges && wave_any(wc != W_NONE)) {
+                const int ux = (int)(wc % 3u) - 1, uy = (int)(wc / 3u % 3u) - 1, uz = (int)(wc / 9u) - 1;
+                if (wc != W_NONE) {
+                    ax = h.x - (float)(ux * Lx);
+                    hy = h.y - (float)(uy * Ly);
+                    hz = h.z - (float)(uz * Lz);
+                    seed = P.seeds[frag_d2i(ux, uy, uz)];
+                    u = S.item[2][k];
+                    v = S.item[3][k];
+                }
+            }
+            PairIn o;
+            pair_kin(o, ax, hy, hz, hv, make_float4(pj.x, pj.y, pj.z, 0.f), make_float4(vj.x, vj.y, vj.z, 0.f));
+            o.x = seed - low_discrepancy((float)(u & 0x3FFu), (float)(int)u, (float)(v & 0x3FFu), (float)(int)v);
+            return o;
+        });
+    }
+
+    // ---- wall pairs: the particles that are not sdf_far and the frozen wall
+    // particles in the 27 cells of the wall cell list around them, as
+    // k_wall_force evaluates them; summed apart
+    if (MOVE == 2 && A.nwall > 0 && wave_any(wnear)) {
+        const UDX_GLOBAL f4v *const wp = (const UDX_GLOBAL f4v *)A.wpos;
+        const UDX_GLOBAL int *const ws = gptr(A.wstarts);
+        Run r1{0, 0, 0, 0, 0, 0, 0, pi.x, false};
+        if (wnear) {
+            auto clampc = [](float x, int W) {
+                const int q = (int)__builtin_floor((double)x + 0.5 * (double)W);
+                return q < 1 ? 1 : (q > W - 2 ? W - 2 : q);
+            };
+            const int c = (clampc(pi.x, A.Wx) - 1) +
+                          A.Wx * ((clampc(pi.y, A.Wy) + dy) + A.Wy * (clampc(pi.z, A.Wz) + dz));
+            r1.j = ws[c];
+            r1.n = ws[c + 3] - r1.j;
+        }
+        const float wseed = *A.wseed;
+        __syncthreads();
+        pass(PassTag<true>{}, r1, r1, false, false, 0, 0, wp, [&](int, unsigned meta, int j) {
+            const unsigned home = meta & 63u;
+            const int ih = first - i0 + (int)home;
+            const float4 h = S.hp[home], hv = S.hv[home];
+            const f3v q = pos_at(wp, (unsigned)j * 16u, 0);
+            float u[3];
+            wvel_at(A.wv, q.x, q.y, q.z, u);
+            PairIn o;
+            pair_kin(o, h.x, h.y, h.z, hv, make_float4(q.x, q.y, q.z, 0.f), make_float4(u[0], u[1], u[2], 0.f));
+            // mean0var1ii(seed, i, wall) (src/math/rnd/dev.h:57-63)
+            o.x = wseed - low_discrepancy((float)(ih & 0x3FF), (float)ih, (float)(j & 0x3FF), (float)j);
+            return o;
+        });
+    }
+
+    if (row < 3) {
+        S.sum[0][row][lane] = acc[0];
+        if (MOVE == 2) S.sum[1][row][lane] = acc[1];
+    }
+    __syncthreads();
+    if (row == 0)
+        finish<MOVE, false>(A, P, active, i + i0, S.hp[lane], S.hv[lane],
+                            make_float3(S.sum[0][0][lane], S.sum[0][1][lane], S.sum[0][2][lane]), wnear,
+                            make_float3(S.sum[1][0][lane], S.sum[1][1][lane], S.sum[1][2][lane]), Stress{});
+}
+
+// at most 72 VGPRs: three blocks of nine waves per CU
+template <int WR, int MOVE>
+__global__ __launch_bounds__(CO_THREADS) __attribute__((amdgpu_waves_per_eu(7))) void k_dpd_coop(DpdK A) {
+    __shared__ CoopLds S;
+    coop_block<WR, MOVE>(A, blockIdx.x * 64, S);
 }
 
 // ---------------------------------------------------------------- half shell
@@ -1329,10 +1851,29 @@ double split_edges = 1048576.0;   // udx_dpd_set_split_edges
 // grid; results are identical either way
 bool split_halo(const DpdLaunch &a) { return a.eidx && a.periodic && edge_estimate(a.box, a.nmax) >= split_edges; }
 
+// One block per 64 particles (k_dpd_coop) while its blocks come to at most
+// twelve per CU.  A lane-per-particle launch is one latency chain long up to
+// about that size; past it the chip has waves enough to hide the chain, and the
+// barriers of the blocks cost more.  Measured, one step with its cell list
+// (lane per particle -> block): density 10, 138 thousand particles 191 -> 140
+// us, 220 thousand 207 -> 191, 328 thousand 228 -> 252; density 5, 240 thousand
+// 165 -> 166; density 3, 144 thousand 129 -> 120, 240 thousand 143 -> 156.
+// Without x slabs a run has twice the candidates, which the blocks test one
+// row to a wave: level at 195 thousand (182 -> 185), so the line is lower.
+bool dpd_small(const DpdK &k, int nmax) { return ceil_div(nmax, 64) <= (k.bstarts ? 12 : 8) * 256; }
+
 template <int WR, bool EXACT>
 int launch_dpd(hipStream_t s, const DpdK &k, int nmax) {
     const dim3 g(ceil_div(nmax, DPD_THREADS)), b(DPD_THREADS);
     const Box box{{k.Lx, k.Ly, k.Lz}};
+    if (dpd_small(k, nmax) && !(k.eidx && k.periodic && edge_estimate(box, nmax) >= split_edges)) {
+        const dim3 gc(ceil_div(nmax, 64)), bc(CO_THREADS);
+        if (k.opos && k.sdf.tex) hipLaunchKernelGGL((k_dpd_coop<WR, 2>), gc, bc, 0, s, k);
+        else if (k.opos) hipLaunchKernelGGL((k_dpd_coop<WR, 1>), gc, bc, 0, s, k);
+        else hipLaunchKernelGGL((k_dpd_coop<WR, 0>), gc, bc, 0, s, k);
+        UDX_LAUNCHED();
+        return UDX_OK;
+    }
     if (k.opos) {
         // the fused move (dpd_move_fused): both force modes give the same bits
         if (k.sdf.tex) hipLaunchKernelGGL((k_dpd<WR, false, PH_ALL, 2>), g, b, 0, s, k);

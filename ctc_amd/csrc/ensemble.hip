@@ -425,7 +425,7 @@ int udx_ens_ini(udx_ctx *ctx, int nbox, const udx_ens_box *boxes, udx_ens **out)
     if (!st) st = dev_alloc(&e->boxL, (size_t)nbox);
     if (!st) st = dev_alloc(&e->mb, (size_t)nbox);
     for (int k = 0; k < 2 && !st; k++) {
-        st = dev_alloc(&e->pos[k], (size_t)e->ntot);
+        st = dev_alloc(&e->pos[k], (size_t)e->ntot + POS_PAD);
         if (!st) st = dev_alloc(&e->vel[k], (size_t)e->ntot);
     }
     if (!st) st = dev_alloc(&e->ff, (size_t)e->ntot);

@@ -126,6 +126,10 @@ void frag_free(FragTables *t);
 // ecount (optional): a box's edge list counter, cleared here for the step
 int frag_build(hipStream_t s, const FragTables *t, const Box &b, const int *starts, int *ecount = nullptr);
 
+// entries a gather may read past a lane's last candidate (values unused): the
+// position streams it reads have this many more than their particles
+constexpr int POS_PAD = 128;
+
 struct DpdLaunch {
     const float4 *pos, *vel;
     const int *starts;      // ncells + 1, starts[ncells] = n

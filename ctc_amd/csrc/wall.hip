@@ -608,7 +608,7 @@ int wall_build_frozen(hipStream_t s, WallSet *w, const SdfField *q, int nw, floa
     st = clist_alloc(&w->cl, wb, ntot > 0 ? ntot : 1);
     float *sorted = nullptr;
     if (!st) st = dev_alloc(&sorted, 6L * (ntot > 0 ? ntot : 1));
-    if (!st) st = dev_alloc(&w->pos, ntot > 0 ? ntot : 1);
+    if (!st) st = dev_alloc(&w->pos, (size_t)ntot + POS_PAD);
     if (!st) st = clist_sort_aos(s, &w->cl, ntot, all);
     if (!st) st = gather_aos(s, &w->cl, ntot, all, sorted);
     if (!st && ntot > 0) {

@@ -1,0 +1,145 @@
+"""The block-per-64-particles force kernel at the sizes where it changes what
+it does, bit for bit against the CPU oracle (the sums have one defined order,
+so no tolerance): a pair list longer than its LDS slots, runs of more than 64
+candidates (taken 64 at a time), runs too long to stage, the smallest periodic
+box, a last block with one particle, whole cells and x slabs, and walls."""
+import sys
+
+import numpy as np
+import pytest
+
+import oracle as O
+from oracle import wall as W
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+if not torch.cuda.is_available():  # pragma: no cover - CPU container
+    pytest.skip("no GPU", allow_module_level=True)
+
+from ctc_amd import udx as U  # noqa: E402
+
+DT = 1e-4
+
+
+def say(*a):
+    print(*a, flush=True)
+    sys.stdout.flush()
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    return U.Context()
+
+
+def host(t):
+    torch.cuda.synchronize()
+    return t.cpu().numpy()
+
+
+def particles(L, n, seed, clump=0.0):
+    """n uniform particles, a share of them in one corner cell and its
+    neighbours across the periodic boundary"""
+    rng = np.random.default_rng(seed)
+    pp = np.zeros((n, 6), np.float32)
+    pp[:, :3] = rng.uniform(-0.5, 0.5, (n, 3)) * np.array(L)
+    k = int(clump * n)
+    half = np.array(L) / 2
+    pp[:k, :3] = (rng.uniform(-0.9, 0.9, (k, 3)) + 2 * half) % (2 * half) - half
+    pp[:, :3] = np.clip(pp[:, :3], -half, np.nextafter(half.astype(np.float32), np.float32(0)))
+    pp[:, 3:] = rng.normal(0, 0.5, (n, 3))
+    return pp
+
+
+# box, particles, share of them around the corner
+CASES = [((3, 3, 3), 81, 0.0),          # every pair wraps or nearly so
+         ((9, 8, 7), 65 * 3, 0.0),      # last block: 3 of 64
+         ((4, 5, 6), 1, 0.0),
+         ((8, 8, 8), 8 * 8 * 8 * 20 + 1, 0.0),    # 64 x 84 pairs a block: two windows; unions above 128
+         ((5, 4, 6), 5 * 4 * 6 * 70, 0.0),        # 210 candidates a run
+         ((12, 11, 13), 12 * 11 * 13 * 2, 0.3)]   # sparse box, one dense corner across the boundary
+
+
+@pytest.mark.parametrize("L,n,clump", CASES)
+@pytest.mark.parametrize("spow", [0.25, 1.0])
+def test_step_bit_exact(ctx, L, n, clump, spow):
+    say("block forces", L, n, clump, spow)
+    pp = particles(L, n, 3, clump)
+    par = (25.0, 4.5, O.dpd_sigma(0.5, 4.5, 1e-3), spow)
+    seeds = O.seeds_table(2)
+    flu = U.Flu(ctx, L, n, U.PairDpd(*par), DT)
+    d = torch.as_tensor(pp).cuda()
+    flu.set_pp(d)
+    flu.run(2, seeds)
+    out = torch.zeros_like(d)
+    flu.get_pp(out)
+    got, npair = host(out), flu.pairs()
+    flu.close()
+    ref, total = pp, 0
+    for k in range(2):
+        ref, p = O.flu_step(L, ref, par, seeds[k], DT, nthreads=8)
+        total += p
+    assert npair == total
+    assert np.array_equal(got.view(np.uint32), ref.view(np.uint32))
+
+
+@pytest.mark.parametrize("L,n,clump", CASES[1:])
+@pytest.mark.parametrize("periodic", [True, False])
+def test_whole_cells_bit_exact(ctx, L, n, clump, periodic):
+    """the module binding: no slab starts, forces added to AoS; also equal to
+    the lane-per-particle kernels (split halo forced)"""
+    say("block forces, whole cells", L, n, clump, periodic)
+    starts, counts, srt, _ = O.clist_build(L, particles(L, n, 4, clump))
+    par = (25.0, 4.5, O.dpd_sigma(0.5, 4.5, 1e-3), 0.25)
+    seeds = O.seeds_table(1)[0]
+    f0 = np.random.default_rng(5).normal(0, 1, (n, 3)).astype(np.float32)
+    want, total = O.dpd_forces(L, srt, starts, counts, par, seeds, periodic=periodic, nthreads=8, ff=f0)
+    f = U.FluForces(ctx, L, n)
+    sd, pd = torch.as_tensor(starts).cuda(), torch.as_tensor(srt).cuda()
+    try:
+        for edges in (1 << 20, 0):
+            U.set_split_edges(edges)
+            f.prepare(pd)
+            ff = torch.as_tensor(f0).cuda()
+            f.pairs(reset=True)
+            f.apply(U.PairDpd(*par), U._ptr(sd), ff, periodic=periodic, seeds=seeds)
+            assert f.pairs() == total // 2
+            assert np.array_equal(host(ff).view(np.uint32), want.view(np.uint32))
+    finally:
+        U.set_split_edges(1 << 20)
+        f.close()
+
+
+@pytest.mark.parametrize("rho", [3, 45])
+def test_walls_bit_exact(ctx, rho):
+    """shearing walls; at density 45 a wall run holds 135 candidates"""
+    L, h = (7, 6, 16), 4.0
+    say("block forces, walls", rho)
+    ext, N = np.array(L, np.float32), (48, 48, 48)
+    D = W.plane_channel_sdf(L, 48, h)
+    q, ref = U.Sdf(ctx, L, ext=ext, N=N, D=D), W.Sdf(L, ext, N, D.ravel())
+    pp = particles(L, rho * 7 * 6 * 16, 6)
+    d = torch.as_tensor(pp).cuda()
+    w = U.Wall(ctx, q, d)
+    n = w.n_solvent
+    cur = host(d)[:n].copy()
+    _, frozen = ref.freeze(pp)
+    wst, _, wpp, _ = O.clist_build(W.margin_box(L), W.wall_images(L, frozen), sub=1)
+    par = (25.0, 4.5, O.dpd_sigma(0.5, 4.5, 1e-3), 0.25)
+    seeds = np.concatenate([O.seeds_table(2), O.kiss_fill(42, 42, 42, 42, 2)[:, None]], axis=1)
+    flu = U.Flu(ctx, L, n, U.PairDpd(*par), DT, 1.0, (0.1, 0.0, 0.0))
+    flu.set_pp(d[:n].contiguous())
+    flu.set_wall(w)
+    flu.run(2, seeds)
+    out = torch.zeros((n, 6), device="cuda")
+    flu.get_pp(out)
+    got, gw = host(out), flu.wall_pairs()
+    flu.close()
+    tw = 0
+    for k in range(2):
+        cur, _, nw = W.flu_wall_step(L, cur, par, seeds[k], DT, ref, wpp, wst, accel=(0.1, 0.0, 0.0), nthreads=8)
+        tw += nw
+    assert gw == tw and tw > 0
+    assert np.array_equal(got.view(np.uint32), cur.view(np.uint32))
+    w.close()
+    q.close()
