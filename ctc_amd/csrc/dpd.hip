@@ -91,6 +91,13 @@ __device__ __forceinline__ UDX_GLOBAL T *gptr(T *p) {
     return (UDX_GLOBAL T *)p;
 }
 
+// x, y, z of the entry at a byte offset, plus K entries folded into the load.
+// The 32-bit offset (indices stay below 2^27) goes into the load beside the
+// base; a signed index takes five more instructions per particle to widen.
+__device__ __forceinline__ f3v pos_at(const UDX_GLOBAL f4v *p, unsigned byte, int k) {
+    return *(const UDX_GLOBAL f3v *)((const UDX_GLOBAL char *)p + (size_t)byte + 16 * k);
+}
+
 struct DpdP {
     const UDX_GLOBAL f4v *pos, *vel;
     const UDX_GLOBAL int *starts, *fss, *bstarts;
@@ -99,11 +106,11 @@ struct DpdP {
     DpdPar par;
     // x, y, z of a particle (w is not used)
     __device__ __forceinline__ float4 p(int j) const {
-        const f3v v = *(const UDX_GLOBAL f3v *)(pos + j);
+        const f3v v = pos_at(pos, (unsigned)j * 16u, 0);
         return make_float4(v.x, v.y, v.z, 0.f);
     }
     __device__ __forceinline__ float4 v(int j) const {
-        const f3v u = *(const UDX_GLOBAL f3v *)(vel + j);
+        const f3v u = pos_at(vel, (unsigned)j * 16u, 0);
         return make_float4(u.x, u.y, u.z, 0.f);
     }
 };
@@ -235,6 +242,29 @@ __device__ __forceinline__ PairIn pair_in_wrapped(const DpdP &P, unsigned ent, i
     return o;
 }
 
+// v summed over the lanes up to this one
+__device__ __forceinline__ int wave_scan_add(int v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);   // row_shr:1
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);   // row_bcast:15
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);   // row_bcast:31
+    return v;
+}
+
+// smallest and largest value over the wave's lanes
+__device__ __forceinline__ int wave_min(int v) {
+    v = min(v, __builtin_amdgcn_update_dpp(0x7fffffff, v, 0x111, 0xf, 0xf, false));
+    v = min(v, __builtin_amdgcn_update_dpp(0x7fffffff, v, 0x112, 0xf, 0xf, false));
+    v = min(v, __builtin_amdgcn_update_dpp(0x7fffffff, v, 0x114, 0xf, 0xf, false));
+    v = min(v, __builtin_amdgcn_update_dpp(0x7fffffff, v, 0x118, 0xf, 0xf, false));
+    v = min(v, __builtin_amdgcn_update_dpp(0x7fffffff, v, 0x142, 0xa, 0xf, false));
+    v = min(v, __builtin_amdgcn_update_dpp(0x7fffffff, v, 0x143, 0xc, 0xf, false));
+    return __builtin_amdgcn_readlane(v, 63);
+}
+__device__ __forceinline__ int wave_max(int v) { return -wave_min(-v); }
+
 // Candidate window along x.  With x-slab starts a row run [x0, x1] of cells
 // (wrap wx) is cut to the slabs that can hold a particle within the cutoff:
 // a candidate at y-z distance >= d from the particle has |dx| < sqrt(1 - d^2).
@@ -251,32 +281,34 @@ __device__ __forceinline__ float row_halfwidth(int dy, int dz, float fy, float f
     gy = fmaxf(gy - WIN_MARGIN, 0.f);
     gz = fmaxf(gz - WIN_MARGIN, 0.f);
     const float w2 = 1.00001f - gy * gy - gz * gz;
-    return w2 < 0.f ? -1.f : __builtin_sqrtf(w2) + WIN_MARGIN;
+    return w2 < 0.f ? -1.f : __builtin_amdgcn_sqrtf(w2) + WIN_MARGIN;
 }
 
-// candidates of the run [x0, x1] of the row starting at cell `base`, for the
-// particle at x = ax in the run's frame: index range [*j, *j + *n)
-__device__ __forceinline__ void run_range(const DpdP &P, int base, int x0, int x1, float ax, float hw, int *j,
+// candidates of the run [x0, x1] of the row starting at cell `base`, for a
+// particle in column c of the run's frame (its own column less the wrap times
+// the box side), fx into its cell: index range [*j, *j + *n).  The window is
+// counted in slabs from the particle's cell, so floats hold it exactly enough
+// for the margin (slabs counted from the box edge need doubles, three times
+// the issue cycles).
+__device__ __forceinline__ void run_range(const DpdP &P, int base, int x0, int x1, int c, float fx, float hw, int *j,
                                           int *n) {
-    if (!P.bstarts) {
-        *j = P.starts[base + x0];
-        *n = P.starts[base + x1 + 1] - *j;
-        return;
+    const UDX_GLOBAL int *st = P.starts;
+    int lo = base + x0, hi = base + x1;
+    if (P.bstarts) {
+        const int S = P.sub;
+        st = P.bstarts;
+        lo = max(c * S + (int)__builtin_floorf((fx - hw) * (float)S), x0 * S);
+        hi = min(c * S + (int)__builtin_floorf((fx + hw) * (float)S), x1 * S + S - 1);
+        if (!(hw >= 0.f) || lo > hi) {
+            *j = 0;
+            *n = 0;
+            return;
+        }
+        lo += base * S;
+        hi += base * S;
     }
-    const int S = P.sub;
-    const double h = 0.5 * (double)P.Lx;
-    double lo = __builtin_floor(((double)ax - (double)hw + h) * (double)S);
-    double hi = __builtin_floor(((double)ax + (double)hw + h) * (double)S);
-    lo = fmax(lo, (double)(x0 * S));
-    hi = fmin(hi, (double)(x1 * S + S - 1));
-    if (!(hw >= 0.f) || lo > hi) {
-        *j = 0;
-        *n = 0;
-        return;
-    }
-    const int sb = base * S;
-    *j = P.bstarts[sb + (int)lo];
-    *n = P.bstarts[sb + (int)hi + 1] - *j;
+    *j = st[lo];
+    *n = st[hi + 1] - *j;
 }
 
 template <bool B>
@@ -406,7 +438,7 @@ __device__ __forceinline__ void dpd_block(const DpdK &A, int first) {
 
     float4 pi = make_float4(0.f, 0.f, 0.f, 0.f), vi = pi;
     int cx = 0, cy = 0, cz = 0, istart = 0;
-    float ry = 0.f, rz = 0.f;   // position inside the cell along y and z
+    float rx = 0.f, ry = 0.f, rz = 0.f;   // position inside the cell
     if (active) {
         pi = P.p(i);
         vi = P.v(i);
@@ -414,6 +446,7 @@ __device__ __forceinline__ void dpd_block(const DpdK &A, int first) {
         cell_coord(pi.y, Ly, &cy);
         cell_coord(pi.z, Lz, &cz);
         istart = P.starts[cx + Lx * (cy + Ly * cz)];
+        rx = (float)((double)pi.x + 0.5 * (double)Lx - (double)cx);
         ry = (float)((double)pi.y + 0.5 * (double)Ly - (double)cy);
         rz = (float)((double)pi.z + 0.5 * (double)Lz - (double)cz);
     }
@@ -449,38 +482,38 @@ __device__ __forceinline__ void dpd_block(const DpdK &A, int first) {
     int gen = 0, gfull = 0;   // next generation; generations below gfull are drained
     const int idle_j = active ? i : P.i0;
     const unsigned idle = (unsigned)idle_j | (W_NONE << 27);
-    auto add = [&](bool v, const float3 &f, const PairIn &pq) {
-        if (v) {
-            fx += f.x;
-            fy += f.y;
-            fz += f.z;
-            if (STRESS) {
-                sxx += 0.5f * f.x * pq.dx;
-                sxy += 0.5f * f.x * pq.dy;
-                sxz += 0.5f * f.x * pq.dz;
-                syy += 0.5f * f.y * pq.dy;
-                syz += 0.5f * f.y * pq.dz;
-                szz += 0.5f * f.z * pq.dz;
-            }
+    auto add = [&](const float3 &f, const PairIn &pq) {
+        fx += f.x;
+        fy += f.y;
+        fz += f.z;
+        if (STRESS) {
+            sxx += 0.5f * f.x * pq.dx;
+            sxy += 0.5f * f.x * pq.dy;
+            sxz += 0.5f * f.x * pq.dz;
+            syy += 0.5f * f.y * pq.dy;
+            syz += 0.5f * f.y * pq.dz;
+            szz += 0.5f * f.z * pq.dz;
         }
     };
-    auto decode = [&](unsigned e) { return gt[e >> OBITS] + (int)(e & OMASK); };
+    auto pair_force = [&](bool live, const PairIn &q, float x) {
+        return dpd_pair<WR, EXACT>(P.par, q.dx, q.dy, q.dz, q.r2, q.dvx, q.dvy, q.dvz, x * R_SQRT2, live);
+    };
+    // (an idle slot reads whatever is in its ring slot, which the select drops)
+    auto decode = [&](bool live, unsigned k) {
+        const unsigned e = *slot(k);
+        const int j = gt[e >> OBITS] + (int)(e & OMASK);
+        return live ? j : idle_j;
+    };
     auto pair_step = [&](auto) {
         const unsigned fl = tail - head;
         const bool va = fl > 0u, vb = fl > STEP;
-        const int ja = va ? decode(*slot(head)) : idle_j;
-        const int jb = vb ? decode(*slot(head + STEP)) : idle_j;
-        const PairIn a = pair_in_bulk_j(P, ja, i, pi, vi, seed_bulk);
-        const PairIn b = pair_in_bulk_j(P, jb, i, pi, vi, seed_bulk);
+        const PairIn a = pair_in_bulk_j(P, decode(va, head), i, pi, vi, seed_bulk);
+        const PairIn b = pair_in_bulk_j(P, decode(vb, head + STEP), i, pi, vi, seed_bulk);
         float xa = a.x, xb = b.x;
         logistic18x2(&xa, &xb);
-        const float3 f1 = dpd_pair<WR, EXACT>(P.par, a.dx, a.dy, a.dz, a.r2, a.dvx, a.dvy, a.dvz, xa * R_SQRT2);
-        const float3 f2 = dpd_pair<WR, EXACT>(P.par, b.dx, b.dy, b.dz, b.r2, b.dvx, b.dvy, b.dvz, xb * R_SQRT2);
-        add(va, f1, a);
-        add(vb, f2, b);
-        const unsigned took = fl < 2u * STEP ? fl : 2u * STEP;
-        head += took;
-        npair += (int)(took / STEP);
+        add(pair_force(va, a, xa), a);
+        add(pair_force(vb, b, xb), b);
+        head += fl < 2u * STEP ? fl : 2u * STEP;
     };
     // room for `need` more entries in every lane (need <= 2 DRAIN_STEPS)
     auto make_room = [&](auto pass, unsigned need) {
@@ -521,15 +554,10 @@ __device__ __forceinline__ void dpd_block(const DpdK &A, int first) {
         int j0 = 0, n0 = 0;
         if (active && yy >= 0 && yy < Ly && zz >= 0 && zz < Lz) {
             const int x0 = cx > 0 ? cx - 1 : 0, x1 = cx + 1 < Lx ? cx + 1 : Lx - 1;
-            run_range(P, Lx * (yy + Ly * zz), x0, x1, pi.x, row_halfwidth(dy, dz, ry, rz), &j0, &n0);
+            run_range(P, Lx * (yy + Ly * zz), x0, x1, cx, rx, row_halfwidth(dy, dz, ry, rz), &j0, &n0);
         }
         // the union of the wave's candidate ranges of this row
-        int lo = n0 > 0 ? j0 : 0x7fffffff, hi = n0 > 0 ? j0 + n0 : 0;
-#pragma unroll
-        for (int d = 32; d >= 1; d >>= 1) {
-            lo = min(lo, __shfl_xor(lo, d, 64));
-            hi = max(hi, __shfl_xor(hi, d, 64));
-        }
+        const int lo = wave_min(n0 > 0 ? j0 : 0x7fffffff), hi = wave_max(n0 > 0 ? j0 + n0 : 0);
         if (hi <= lo) return;
         // candidate k of the lane's range is i itself (own row only)
         const int kself = SELF ? i - j0 : -1;
@@ -589,6 +617,7 @@ __device__ __forceinline__ void dpd_block(const DpdK &A, int first) {
         bulk_row(4, PassTag<true>{});
         for (int row = 5; row < 9; row++) bulk_row(row, PassTag<false>{});
         drain(PassTag<true>{});
+        npair = (int)(tail / STEP);   // every entry queued was a pair
     }
 
     // ---- halo pass: the cells across the periodic boundary.  The noise
@@ -639,10 +668,8 @@ __device__ __forceinline__ void dpd_block(const DpdK &A, int first) {
             const PairIn b = pair_in_wrapped(P, eb, (int)ub, (int)xb_, pi, vi);
             float xa = a.x, xb = b.x;
             logistic18x2(&xa, &xb);
-            const float3 f1 = dpd_pair<WR, EXACT>(P.par, a.dx, a.dy, a.dz, a.r2, a.dvx, a.dvy, a.dvz, xa * R_SQRT2);
-            const float3 f2 = dpd_pair<WR, EXACT>(P.par, b.dx, b.dy, b.dz, b.r2, b.dvx, b.dvy, b.dvz, xb * R_SQRT2);
-            add(va, f1, a);
-            add(vb, f2, b);
+            add(pair_force(va, a, xa), a);
+            add(pair_force(vb, b, xb), b);
             const unsigned took = fl < 2u * HSTEP ? fl : 2u * HSTEP;
             hh += took;
             npair += (int)(took / HSTEP);
@@ -680,11 +707,11 @@ __device__ __forceinline__ void dpd_block(const DpdK &A, int first) {
                 const float hw = row_halfwidth(dy, dz, ry, rz);
                 const int base = Lx * (yy + Ly * zz);
                 if (xrun(0, cx, Lx, &x0, &x1, &wx0) && (yzwrap || wx0 != 0)) {
-                    run_range(P, base, x0, x1, pi.x - (float)(wx0 * Lx), hw, &j0, &n0);
+                    run_range(P, base, x0, x1, cx - wx0 * Lx, rx, hw, &j0, &n0);
                     if (n0 > 0) runtab(wx0, x0, &aid0, &b0, &m0);
                 }
                 if (xrun(1, cx, Lx, &x0, &x1, &wx1) && (yzwrap || wx1 != 0)) {
-                    run_range(P, base, x0, x1, pi.x - (float)(wx1 * Lx), hw, &j1, &n1);
+                    run_range(P, base, x0, x1, cx - wx1 * Lx, rx, hw, &j1, &n1);
                     if (n1 > 0) runtab(wx1, x0, &aid1, &b1, &m1);
                 }
             }
@@ -909,22 +936,6 @@ constexpr int CO_STAGE = 128;               // candidates a wave stages in LDS
 constexpr int CO_CAP = 3072;                // pair slots of a block (density 10 has about 2600)
 constexpr unsigned CO_DENSE = 0xFFu;        // a row with more than 64 candidates in a run
 
-// v summed over the lanes up to this one
-__device__ __forceinline__ int wave_scan_add(int v) {
-    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);   // row_shr:1
-    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);   // row_bcast:15
-    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);   // row_bcast:31
-    return v;
-}
-
-// x, y, z of particle j + K, K a constant folded into the load
-__device__ __forceinline__ f3v pos_at(const UDX_GLOBAL f4v *p, unsigned byte, int k) {
-    return *(const UDX_GLOBAL f3v *)((const UDX_GLOBAL char *)p + (size_t)byte + 16 * k);
-}
-
 // hits of up to 64 candidates as bits, candidate k at bit 31 - (k mod 32) of
 // word k / 32: the sign of r2 - 1, shifted in from the right.  at(k) reads the
 // lane's candidate k, for k up to seven past the last one.
@@ -964,18 +975,6 @@ __device__ __forceinline__ Mask64 test64(int n, float ax, float ay, float az, At
     }
     return m;
 }
-
-// smallest and largest value over the wave's lanes
-__device__ __forceinline__ int wave_min(int v) {
-    v = min(v, __builtin_amdgcn_update_dpp(0x7fffffff, v, 0x111, 0xf, 0xf, false));
-    v = min(v, __builtin_amdgcn_update_dpp(0x7fffffff, v, 0x112, 0xf, 0xf, false));
-    v = min(v, __builtin_amdgcn_update_dpp(0x7fffffff, v, 0x114, 0xf, 0xf, false));
-    v = min(v, __builtin_amdgcn_update_dpp(0x7fffffff, v, 0x118, 0xf, 0xf, false));
-    v = min(v, __builtin_amdgcn_update_dpp(0x7fffffff, v, 0x142, 0xa, 0xf, false));
-    v = min(v, __builtin_amdgcn_update_dpp(0x7fffffff, v, 0x143, 0xc, 0xf, false));
-    return __builtin_amdgcn_readlane(v, 63);
-}
-__device__ __forceinline__ int wave_max(int v) { return -wave_min(-v); }
 
 struct CoopLds {
     float4 hp[64], hv[64];
@@ -1273,28 +1272,11 @@ __device__ __forceinline__ void coop_block(const DpdK &A, int first, CoopLds &S)
                         (xrun(1, cx, Lx, &r2.x0, &r2.x1, &r2.wx) && r2.wx != 0);
             }
         }
-        // candidates of the run's cells within reach along x: cut to x slabs where the list has them
         auto range = [&](Run &r) {
             r.ax = pi.x - (float)(r.wx * Lx);
-            int lo, hi;
-            const UDX_GLOBAL int *st = P.bstarts;
-            if (!st) {
-                st = P.starts;
-                lo = base + r.x0;
-                hi = base + r.x1;
-            } else {
-                const int c = (cx - r.wx * Lx) * P.sub;
-                lo = c + (int)__builtin_floorf((rx - hw) * (float)P.sub);
-                hi = c + (int)__builtin_floorf((rx + hw) * (float)P.sub);
-                lo = max(lo, r.x0 * P.sub);
-                hi = min(hi, r.x1 * P.sub + P.sub - 1);
-                r.on = r.on && lo <= hi;
-                lo += base * P.sub;
-                hi += base * P.sub;
-            }
-            const int a = st[r.on ? lo : 0], e = st[r.on ? hi + 1 : 0];
-            r.n = e - a;
-            r.j = r.n > 0 ? a - i0 : 0;
+            if (r.on) run_range(P, base, r.x0, r.x1, cx - r.wx * Lx, rx, hw, &r.j, &r.n);
+            r.on = r.n > 0;
+            r.j = r.on ? r.j - i0 : 0;
         };
         auto lists = [&](Run &r) {
             const int fid = frag_d2i(r.wx, wy, wz), anti = frag_d2i(-r.wx, -wy, -wz);
@@ -1461,7 +1443,7 @@ __device__ __forceinline__ void dpd_half_block(const DpdK &A, int first, HsWave 
 
     float4 pi = make_float4(0.f, 0.f, 0.f, 0.f), vi = pi;
     int cx = 0, cy = 0, cz = 0, istart = 0;
-    float ry = 0.f, rz = 0.f;
+    float rx = 0.f, ry = 0.f, rz = 0.f;
     if (active) {
         pi = P.p(i);
         vi = P.v(i);
@@ -1469,6 +1451,7 @@ __device__ __forceinline__ void dpd_half_block(const DpdK &A, int first, HsWave 
         cell_coord(pi.y, Ly, &cy);
         cell_coord(pi.z, Lz, &cz);
         istart = P.starts[cx + Lx * (cy + Ly * cz)];
+        rx = (float)((double)pi.x + 0.5 * (double)Lx - (double)cx);
         ry = (float)((double)pi.y + 0.5 * (double)Ly - (double)cy);
         rz = (float)((double)pi.z + 0.5 * (double)Lz - (double)cz);
     }
@@ -1536,15 +1519,10 @@ __device__ __forceinline__ void dpd_half_block(const DpdK &A, int first, HsWave 
         if (active && yy >= 0 && yy < Ly && zz >= 0) {
             const int x0 = cx > 0 ? cx - 1 : 0;
             const int x1 = row == 4 ? cx : (cx + 1 < Lx ? cx + 1 : Lx - 1);
-            run_range(P, Lx * (yy + Ly * zz), x0, x1, pi.x, row_halfwidth(dy, dz, ry, rz), &j0, &n0);
+            run_range(P, Lx * (yy + Ly * zz), x0, x1, cx, rx, row_halfwidth(dy, dz, ry, rz), &j0, &n0);
             if (row == 4) n0 = max(0, min(n0, i - j0));   // own row: lower indices only
         }
-        int lo = n0 > 0 ? j0 : 0x7fffffff, hi = n0 > 0 ? j0 + n0 : 0;
-#pragma unroll
-        for (int d = 32; d >= 1; d >>= 1) {
-            lo = min(lo, __shfl_xor(lo, d, 64));
-            hi = max(hi, __shfl_xor(hi, d, 64));
-        }
+        const int lo = wave_min(n0 > 0 ? j0 : 0x7fffffff), hi = wave_max(n0 > 0 ? j0 + n0 : 0);
         for (int c0 = lo; c0 < hi; c0 += HS_SC) {
             const int len = min(HS_SC, hi - c0);
             __builtin_amdgcn_wave_barrier();
@@ -1647,9 +1625,9 @@ __device__ __forceinline__ void dpd_half_block(const DpdK &A, int first, HsWave 
                 const float hw = row_halfwidth(dy, dz, ry, rz);
                 const int base = Lx * (yy + Ly * zz);
                 if (xrun(0, cx, Lx, &x0, &x1, &wx0) && (yzwrap || wx0 != 0))
-                    run_range(P, base, x0, x1, pi.x - (float)(wx0 * Lx), hw, &j0, &n0);
+                    run_range(P, base, x0, x1, cx - wx0 * Lx, rx, hw, &j0, &n0);
                 if (xrun(1, cx, Lx, &x0, &x1, &wx1) && (yzwrap || wx1 != 0))
-                    run_range(P, base, x0, x1, pi.x - (float)(wx1 * Lx), hw, &j1, &n1);
+                    run_range(P, base, x0, x1, cx - wx1 * Lx, rx, hw, &j1, &n1);
             }
             const float ay = pi.y - (float)(wy * Ly), az = pi.z - (float)(wz * Lz);
             const float ax0 = pi.x - (float)(wx0 * Lx), ax1 = pi.x - (float)(wx1 * Lx);

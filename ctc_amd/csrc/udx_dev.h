@@ -206,10 +206,12 @@ struct DpdPar { float a, g, s, spow; };
 // reference's fast-math r2 rsqrtf(r2) is 1e-3 wrong in w_R near the cutoff,
 // where w_R = (1 - r)^spow has an unbounded slope).  The template argument
 // EXACT is kept for the generic exponent (powf).  A pair that is no pair (an
-// idle slot, r2 >= 1) gives a value to be discarded, NaN among them.
+// idle slot, r2 >= 1) gives a value to be discarded, NaN among them; a particle
+// against itself with live = false gives a zero that can be added (a sum that
+// starts at +0 keeps its bits).
 template <int WR, bool EXACT>
 __device__ __forceinline__ float3 dpd_pair(const DpdPar &p, float dx, float dy, float dz, float r2,
-                                           float dvx, float dvy, float dvz, float rnd) {
+                                           float dvx, float dvy, float dvz, float rnd, bool live = true) {
     // selects, not branches: a wave nearly always holds both kinds of pairs
     // or none of the close ones
     const bool close = r2 < 1e-6f;
@@ -223,6 +225,7 @@ __device__ __forceinline__ float3 dpd_pair(const DpdPar &p, float dx, float dy, 
     const float wr = wr_pow<WR, EXACT>(rm, p.spow);
     float f0 = __builtin_fmaf(-p.g * wr, ev, p.s * rnd) * wr;
     f0 = __builtin_fmaf(p.a, rm, f0);
+    f0 = live ? f0 : 0.0f;
     return make_float3(f0 * ex, f0 * ey, f0 * ez);
 }
 
