@@ -293,8 +293,7 @@ int udx_clist_fin(udx_clist *c) {
 int udx_clist_build(udx_clist *c, int n, const float *pp, float *ppout, int *nout) {
     UDX_CHECK(c, UDX_EINVAL, "udx_clist_build: null clist");
     hipStream_t s = c->ctx->stream;
-    UDX_TRY(clist_sort_aos(s, &c->c, n, pp));
-    if (ppout) UDX_TRY(gather_aos(s, &c->c, n, pp, ppout));
+    UDX_TRY(clist_sort_aos(s, &c->c, n, pp, ppout));
     if (nout) {
         UDX_HIP(hipMemcpyAsync(nout, c->c.starts + c->c.box.ncells(), sizeof(int), hipMemcpyDeviceToHost, s));
         UDX_HIP(hipStreamSynchronize(s));
@@ -651,10 +650,12 @@ static int flu_step(udx_flu *f, const float *seeds_dev, const float *fsi_seeds, 
     udx_flu::Membranes &m = f->mb;
     const int nvtx = m.nc * m.nv;
     if (f->evk) UDX_HIP(hipEventRecord(f->evk[0], s));
-    if (f->counted) UDX_TRY(clist_finish(s, &f->cl, f->n));
-    else UDX_TRY(clist_sort(s, &f->cl, f->n, f->pos[a]));
-    UDX_TRY(gather_f4(s, &f->cl, f->n, f->pos[a], f->vel[a], f->pos[b], f->vel[b]));
-    UDX_TRY(frag_build(s, &f->frag, f->box, f->cl.starts, f->ecount));
+    if (!f->counted) UDX_TRY(clist_count_only(s, &f->cl, f->n, f->pos[a]));
+    UDX_TRY(clist_finish_f4(s, &f->cl, f->n, f->pos[a], f->vel[a], f->pos[b], f->vel[b]));
+    // (a captured step finds its seeds in the run's table itself)
+    StepSeeds q;
+    if (f->step_stream) q = StepSeeds{f->seeds_dev, f->step_dev, f->seeds_cur, NSEED};
+    UDX_TRY(frag_build(s, &f->frag, f->box, f->cl.starts, f->ecount, q));
     if (m.r) UDX_TRY(rbc_redistribute(s, f->box, m.nc, m.nv, m.pp, m.tmp, m.cfid, m.cnew));
     const bool bounce = m.r && m.bb;
     // objects_save_mesh (src/sim/imp/run.h:30-31): the vertices at the start of the step
@@ -788,19 +789,6 @@ static int flu_step(udx_flu *f, const float *seeds_dev, const float *fsi_seeds, 
     return UDX_OK;
 }
 
-namespace {
-// the seeds of step *step from the run's table, then the counter advanced to
-// the next step (one wave: every lane reads the counter before lane 0 writes
-// it; nothing else in the step reads it)
-__global__ void k_flu_seeds(const float *table, int *step, float *cur) {
-    const int k = threadIdx.x;
-    const int st = *step;
-    if (k < NSEED) cur[k] = table[(long)st * NSEED + k];
-    __syncthreads();
-    if (k == 0) *step = st + 1;
-}
-}  // namespace
-
 static void flu_drop_graph(udx_flu *f) {
     if (f->gexec) (void)hipGraphExecDestroy(f->gexec);
     if (f->graph) (void)hipGraphDestroy(f->graph);
@@ -826,9 +814,7 @@ static int flu_capture(udx_flu *f) {
     UDX_HIP(hipStreamBeginCapture(f->gs, hipStreamCaptureModeThreadLocal));
     int st = UDX_OK;
     for (int k = 0; k < 2 && !st; k++) {
-        hipLaunchKernelGGL(k_flu_seeds, dim3(1), dim3(64), 0, f->gs, f->seeds_dev, f->step_dev, f->seeds_cur);
-        st = hipGetLastError() == hipSuccess ? UDX_OK : UDX_EHIP;
-        if (!st) st = flu_step(f, f->seeds_cur, nullptr, nullptr);
+        st = flu_step(f, f->seeds_cur, nullptr, nullptr);
     }
     hipGraph_t g = nullptr;
     const hipError_t ce = hipStreamEndCapture(f->gs, &g);

@@ -208,14 +208,14 @@ __device__ __forceinline__ PairIn pair_in_halo(const DpdK &A, const DpdP &P, uns
     const int wx = (int)(w % 3u) - 1, wy = (int)((w / 3u) % 3u) - 1, wz = (int)(w / 9u) - 1;
     const float ax = pi.x - (float)(wx * Lx), ay = pi.y - (float)(wy * Ly), az = pi.z - (float)(wz * Lz);
     const int fid = frag_d2i(wx, wy, wz), anti = frag_d2i(-wx, -wy, -wz);
-    const int aid = P.fss[A.foff[fid] + frag_cell(wx, wy, wz, cx, cy, cz, Lx, Ly)] - P.fss[A.foff[fid]] + (i - istart);
+    const int aid = P.fss[A.foff[fid] + frag_cell(wx, wy, wz, cx, cy, cz, Lx, Ly)] + (i - istart);
     int jx = 0, jy = 0, jz = 0;
     cell_coord(pj.x, Lx, &jx);
     cell_coord(pj.y, Ly, &jy);
     cell_coord(pj.z, Lz, &jz);
     const int jstart = P.starts[jx + Lx * (jy + Ly * jz)];
     const int bid =
-        P.fss[A.foff[anti] + frag_cell(-wx, -wy, -wz, jx, jy, jz, Lx, Ly)] - P.fss[A.foff[anti]] + (j - jstart);
+        P.fss[A.foff[anti] + frag_cell(-wx, -wy, -wz, jx, jy, jz, Lx, Ly)] + (j - jstart);
     const bool mask = fid < anti;
     const int u = mask ? aid : bid, v = mask ? bid : aid;
     PairIn o;
@@ -763,8 +763,8 @@ __device__ __forceinline__ void dpd_block(const DpdK &A, int first) {
             auto runtab = [&](int wx, int xs, int *aid, int *bb, bool *mk) {
                 const int fid = frag_d2i(wx, wy, wz), anti = frag_d2i(-wx, -wy, -wz);
                 const int fo = A.foff[fid], ao = A.foff[anti];
-                *aid = P.fss[fo + frag_cell(wx, wy, wz, cx, cy, cz, Lx, Ly)] - P.fss[fo] + (i - istart);
-                *bb = P.fss[ao + frag_cell(-wx, -wy, -wz, xs, yy, zz, Lx, Ly)] - P.fss[ao] -
+                *aid = P.fss[fo + frag_cell(wx, wy, wz, cx, cy, cz, Lx, Ly)] + (i - istart);
+                *bb = P.fss[ao + frag_cell(-wx, -wy, -wz, xs, yy, zz, Lx, Ly)] -
                       P.starts[xs + Lx * (yy + Ly * zz)];
                 *mk = fid < anti;
             };
@@ -1349,8 +1349,8 @@ __device__ __forceinline__ void coop_block(const DpdK &A, int first, CoopLds &S)
             const int fid = frag_d2i(r.wx, wy, wz), anti = frag_d2i(-r.wx, -wy, -wz);
             const int fo = A.foff[fid], ao = A.foff[anti];
             const int hs = P.starts[cx + Lx * (cy + Ly * cz)] - i0;
-            r.aid = P.fss[fo + frag_cell(r.wx, wy, wz, cx, cy, cz, Lx, Ly)] - P.fss[fo] + (i - hs);
-            r.bb = P.fss[ao + frag_cell(-r.wx, -wy, -wz, r.x0, yy, zz, Lx, Ly)] - P.fss[ao] -
+            r.aid = P.fss[fo + frag_cell(r.wx, wy, wz, cx, cy, cz, Lx, Ly)] + (i - hs);
+            r.bb = P.fss[ao + frag_cell(-r.wx, -wy, -wz, r.x0, yy, zz, Lx, Ly)] -
                    (P.starts[r.x0 + base] - i0);
         };
         range(r1);
@@ -1785,30 +1785,115 @@ __global__ __launch_bounds__(256) void k_acc_to_ff(int nmax, const int *n_dev, i
     }
 }
 
-// Counts of the cells of the 26 fragments in fragment-cell order (x
-// fastest, src/exch/flu/dev/map.h:22-42), one extra 0 after each fragment.
-// An exclusive scan over this array gives every fragment's packed-list
-// offsets (src/exch/flu/dev/map.h:44-98) as differences G[off + h] - G[off].
-// The box's edge list counter (if any) starts the step at zero here.
-__global__ __launch_bounds__(256) void k_frag_counts(const int *starts, int Lx, int Ly, int Lz, FragOff fo,
-                                                     int *cnt, int *ecount) {
+// the fragments' cells in fragment-cell order (x fastest,
+// src/exch/flu/dev/map.h:22-42): count of cell h of fragment f
+struct FragCells {
+    const int *starts;
+    int Lx, Ly, x0, y0, z0, ex, ey, n;
+    __device__ __forceinline__ FragCells(const int *st, int lx, int ly, int lz, int f) {
+        const int dx = (f + 2) % 3 - 1, dy = (f / 3 + 2) % 3 - 1, dz = (f / 9 + 2) % 3 - 1;
+        starts = st;
+        Lx = lx;
+        Ly = ly;
+        x0 = dx == 1 ? lx - 1 : 0;
+        y0 = dy == 1 ? ly - 1 : 0;
+        z0 = dz == 1 ? lz - 1 : 0;
+        ex = dx ? 1 : lx;
+        ey = dy ? 1 : ly;
+        n = ex * ey * (dz ? 1 : lz);
+    }
+    __device__ __forceinline__ int operator()(int h) const {
+        const int r = h / ex, cid = x0 + h % ex + Lx * (y0 + r % ey + Ly * (z0 + r / ey));
+        return starts[cid + 1] - starts[cid];
+    }
+};
+
+// Packed-list offsets of one fragment's cells: the exclusive sums of the
+// counts of its n cells (src/exch/flu/dev/map.h:44-98), by one block, NT
+// threads of four cells each and as many rounds as the fragment takes.  A
+// fragment is a face, edge or corner of the box, so its sums need no other
+// block: one launch of 26 blocks where the counts and a scan over all
+// fragments took two or three (16^3: 11.5 -> 3.9 us).
+template <int NT, class Count>
+__device__ __forceinline__ void frag_table(int n, const Count &count, int *fss) {
+    __shared__ int lw[NT / 64];
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    int carry = 0;
+    for (int b = 0; b < n; b += 4 * NT) {
+        const int h0 = b + 4 * tid;
+        int v[4], s = 0;
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            v[u] = h0 + u < n ? count(h0 + u) : 0;
+            s += v[u];
+        }
+        const int inc = wave_scan_add(s);
+        if (lane == 63) lw[w] = inc;
+        __syncthreads();
+        int run = carry + inc - s, all = 0;
+#pragma unroll
+        for (int k = 0; k < NT / 64; k++) {
+            run += k < w ? lw[k] : 0;
+            all += lw[k];
+        }
+        carry += all;
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            if (h0 + u < n) fss[h0 + u] = run;
+            run += v[u];
+        }
+        __syncthreads();
+    }
+}
+
+// Faces of more than FRAG_FACE cells are counted by a launch of their own: the
+// cells of an x face lie a row apart, a cache line each, more than one CU
+// fetches in good time (96^2 faces: 44 us for the one launch).
+constexpr int FRAG_FACE = 4096;
+__global__ __launch_bounds__(256) void k_frag_counts(const int *starts, int Lx, int Ly, int Lz, FragOff fo, int *cnt) {
     const int g = blockIdx.x * blockDim.x + threadIdx.x;
-    if (g == 0 && ecount) *ecount = 0;
     if (g >= fo.off[26]) return;
     int f = 0;
     while (f < 25 && g >= fo.off[f + 1]) f++;
+    const FragCells c(starts, Lx, Ly, Lz, f);
     const int h = g - fo.off[f];
-    const int dx = (f + 2) % 3 - 1, dy = (f / 3 + 2) % 3 - 1, dz = (f / 9 + 2) % 3 - 1;
-    const int ex = dx ? 1 : Lx, ey = dy ? 1 : Ly, ez = dz ? 1 : Lz;
-    int v = 0;
-    if (h < ex * ey * ez) {
-        const int x = (dx == 1 ? Lx - 1 : 0) + h % ex;
-        const int y = (dy == 1 ? Ly - 1 : 0) + (h / ex) % ey;
-        const int z = (dz == 1 ? Lz - 1 : 0) + h / (ex * ey);
-        const int cid = x + Lx * (y + Ly * z);
-        v = starts[cid + 1] - starts[cid];
+    if (h < c.n) cnt[g] = c(h);
+}
+
+// the box's tables, one block per fragment; the first block also clears the
+// box's edge list counter (if any) and, in a captured step, copies the step's
+// seeds from the run's table and advances the step counter
+__global__ __launch_bounds__(1024) void k_frag_tables(const int *starts, int Lx, int Ly, int Lz, FragOff fo,
+                                                      const int *cnt, int *fss, int *ecount, StepSeeds q) {
+    if (blockIdx.x == 0) {
+        if (threadIdx.x == 0 && ecount) *ecount = 0;
+        if (q.table) {
+            const int st = *q.step;
+            __syncthreads();
+            if ((int)threadIdx.x < q.nseed) q.cur[threadIdx.x] = q.table[(long)st * q.nseed + threadIdx.x];
+            if (threadIdx.x == 0) *q.step = st + 1;
+        }
     }
-    cnt[g] = v;
+    const FragCells c(starts, Lx, Ly, Lz, blockIdx.x);
+    const int off = fo.off[blockIdx.x];
+    if (cnt) frag_table<1024>(c.n, [&](int h) { return cnt[off + h]; }, fss + off);
+    else frag_table<1024>(c.n, c, fss + off);
+}
+
+// the same for every box of a batch, 26 blocks a box; the first blocks also
+// copy the step's seeds of every box and clear the edge list counters (the
+// step counter advances later in the step)
+__global__ __launch_bounds__(256) void k_frag_tables_batch(int nbox, const int *fbase, const int *foff,
+                                                           const int *coff, const int4 *boxL, const int *starts,
+                                                           int *fss, int *ecount, const float *table,
+                                                           const int *step, float *seeds) {
+    const int g = blockIdx.x * 256 + threadIdx.x;
+    if (g < 27 * nbox) seeds[g] = table[(long)*step * 27 * nbox + g];
+    if (g < nbox) ecount[g] = 0;
+    const int b = blockIdx.x / 26, f = blockIdx.x % 26;
+    const int4 L = boxL[b];
+    const FragCells c(starts + coff[b], L.x, L.y, L.z, f);
+    frag_table<256>(c.n, c, fss + fbase[b] + foff[27 * b + f]);
 }
 
 DpdK make_k(const DpdLaunch &a) {
@@ -1947,25 +2032,38 @@ int frag_alloc(FragTables *t, const Box &b) {
     }
     t->off[26] = off;
     t->size = off;
-    UDX_TRY(dev_alloc(&t->cnt, off));
     UDX_TRY(dev_alloc(&t->fss, off + 1));
-    UDX_TRY(dev_alloc(&t->scan_tmp, scan_scratch_size(off)));
+    const long xy = (long)b.L[0] * b.L[1], yz = (long)b.L[1] * b.L[2], zx = (long)b.L[2] * b.L[0];
+    if (xy > FRAG_FACE || yz > FRAG_FACE || zx > FRAG_FACE) UDX_TRY(dev_alloc(&t->cnt, off));
     return UDX_OK;
 }
 
 void frag_free(FragTables *t) {
-    dev_free(t->cnt);
     dev_free(t->fss);
-    dev_free(t->scan_tmp);
+    dev_free(t->cnt);
 }
 
-int frag_build(hipStream_t s, const FragTables *t, const Box &b, const int *starts, int *ecount) {
+int frag_build(hipStream_t s, const FragTables *t, const Box &b, const int *starts, int *ecount,
+               const StepSeeds &seeds) {
     FragOff fo;
     for (int f = 0; f < 27; f++) fo.off[f] = t->off[f];
-    hipLaunchKernelGGL(k_frag_counts, dim3(ceil_div(t->size, 256)), dim3(256), 0, s, starts, b.L[0], b.L[1],
-                       b.L[2], fo, t->cnt, ecount);
+    if (t->cnt) {
+        hipLaunchKernelGGL(k_frag_counts, dim3(ceil_div(t->size, 256)), dim3(256), 0, s, starts, b.L[0], b.L[1],
+                           b.L[2], fo, t->cnt);
+        UDX_LAUNCHED();
+    }
+    hipLaunchKernelGGL(k_frag_tables, dim3(26), dim3(1024), 0, s, starts, b.L[0], b.L[1], b.L[2], fo, t->cnt, t->fss,
+                       ecount, seeds);
     UDX_LAUNCHED();
-    return scan_exclusive(s, t->cnt, t->size, t->fss, t->scan_tmp);
+    return UDX_OK;
+}
+
+int frag_build_batch(hipStream_t s, int nbox, const int *fbase, const int *foff, const int *coff, const int4 *boxL,
+                     const int *starts, int *fss, int *ecount, const float *table, const int *step, float *seeds) {
+    hipLaunchKernelGGL(k_frag_tables_batch, dim3(26 * nbox), dim3(256), 0, s, nbox, fbase, foff, coff, boxL, starts,
+                       fss, ecount, table, step, seeds);
+    UDX_LAUNCHED();
+    return UDX_OK;
 }
 
 // mode UDX_MODE_EXACT selects correctly rounded sqrt/division in the pair force

@@ -63,37 +63,6 @@ __global__ __launch_bounds__(256) void k_ens_count(int n, int nbox, const int *p
                     coff[b] * SOLVENT_SUB);
 }
 
-// cell counts of the 26 fragments of every box (as k_frag_counts); the
-// first threads also copy the step's seeds of every box from the run's table
-// and clear the boxes' edge list counters
-__global__ __launch_bounds__(256) void k_ens_frag_counts(int total, int nbox, const int *fbase, const int *foff,
-                                                         const int *coff, const int4 *boxL, const int *starts,
-                                                         int *cnt, const float *table, const int *step,
-                                                         float *seeds, int *ecount) {
-    const int g = blockIdx.x * blockDim.x + threadIdx.x;
-    if (g < 27 * nbox) seeds[g] = table[(long)*step * 27 * nbox + g];
-    if (g < nbox) ecount[g] = 0;
-    if (g >= total) return;
-    const int b = find_box(fbase, nbox, g);
-    const int4 L = boxL[b];
-    const int *off = foff + 27 * b;
-    const int gl = g - fbase[b];
-    int f = 0;
-    while (f < 25 && gl >= off[f + 1]) f++;
-    const int h = gl - off[f];
-    const int dx = (f + 2) % 3 - 1, dy = (f / 3 + 2) % 3 - 1, dz = (f / 9 + 2) % 3 - 1;
-    const int ex = dx ? 1 : L.x, ey = dy ? 1 : L.y, ez = dz ? 1 : L.z;
-    int v = 0;
-    if (h < ex * ey * ez) {
-        const int x = (dx == 1 ? L.x - 1 : 0) + h % ex;
-        const int y = (dy == 1 ? L.y - 1 : 0) + (h / ex) % ey;
-        const int z = (dz == 1 ? L.z - 1 : 0) + h / (ex * ey);
-        const int cid = coff[b] + x + L.x * (y + L.y * z);
-        v = starts[cid + 1] - starts[cid];
-    }
-    cnt[g] = v;
-}
-
 struct MoveBox {
     float Lx, Ly, Lz, dt;
     float mass, ax, ay, az;
@@ -172,7 +141,7 @@ struct udx_ens {
     int *ecount, *eidx;            // edge lists of the gather's halo pass (a counter per box)
     float4 *ef;
     ClistBufs cl;
-    int *fcnt, *fss, *fscan;
+    int *fss;
     float *seeds_table, *seeds_cur, *seeds_host;
     int *step;
     unsigned long long *pairs;
@@ -248,14 +217,9 @@ static int ens_step(udx_ens *e, int cur, int *next) {
     hipStream_t s = e->s;
     const int a = cur, b = 1 - cur, n = e->ntot;
     if (!e->counted) UDX_TRY(ens_count(e, a));
-    UDX_TRY(clist_finish(s, &e->cl, n));
-    UDX_TRY(gather_f4(s, &e->cl, n, e->pos[a], e->vel[a], e->pos[b], e->vel[b]));
-    const int nf = e->ftot > 27 * e->nbox ? e->ftot : 27 * e->nbox;
-    hipLaunchKernelGGL(k_ens_frag_counts, dim3(ceil_div(nf, 256)), dim3(256), 0, s, e->ftot, e->nbox, e->fbase,
-                       e->foff, e->coff, e->boxL, e->cl.starts, e->fcnt, e->seeds_table, e->step, e->seeds_cur,
-                       e->ecount);
-    UDX_LAUNCHED();
-    UDX_TRY(scan_exclusive(s, e->fcnt, e->ftot, e->fss, e->fscan));
+    UDX_TRY(clist_finish_f4(s, &e->cl, n, e->pos[a], e->vel[a], e->pos[b], e->vel[b]));
+    UDX_TRY(frag_build_batch(s, e->nbox, e->fbase, e->foff, e->coff, e->boxL, e->cl.starts, e->fss, e->ecount,
+                             e->seeds_table, e->step, e->seeds_cur));
     UDX_TRY(dpd_forces_batch(s, e->batch[b], e->mode, e->variant));
     const bool fused = e->mode != UDX_MODE_HALF;
     if (!fused) {
@@ -351,9 +315,7 @@ int udx_ens_fin(udx_ens *e) {
     dev_free(e->foff);
     dev_free(e->boxL);
     dev_free(e->mb);
-    dev_free(e->fcnt);
     dev_free(e->fss);
-    dev_free(e->fscan);
     dev_free(e->seeds_table);
     dev_free(e->seeds_cur);
     dev_free(e->step);
@@ -436,9 +398,7 @@ int udx_ens_ini(udx_ctx *ctx, int nbox, const udx_ens_box *boxes, udx_ens **out)
     if (!st) st = dev_alloc(&e->eidx, (size_t)(e->ntot > 0 ? e->ntot : 1));
     if (!st) st = dev_alloc(&e->ef, (size_t)(e->ntot > 0 ? e->ntot : 1));
     if (!st) st = clist_alloc(&e->cl, Box{{e->ctot, 1, 1}}, e->ntot > 0 ? e->ntot : 1, SOLVENT_SUB);
-    if (!st) st = dev_alloc(&e->fcnt, (size_t)e->ftot);
     if (!st) st = dev_alloc(&e->fss, (size_t)e->ftot + 1);
-    if (!st) st = dev_alloc(&e->fscan, (size_t)scan_scratch_size(e->ftot));
     if (!st) st = dev_alloc(&e->seeds_cur, 27 * (size_t)nbox);
     if (!st) st = dev_alloc(&e->step, 1);
     if (!st) st = dev_alloc(&e->pairs, 1);

@@ -476,8 +476,7 @@ int fsi_forces(hipStream_t s, FsiBufs *f, int ns, const float4 *spos, const floa
     UDX_LAUNCHED();
     // at most 7 images per vertex (faces, edges, corner of its outside axes)
     const int nmax = 8 * no;
-    UDX_TRY(clist_sort_aos(s, &f->cl, nmax, f->inst));
-    UDX_TRY(gather_aos(s, &f->cl, nmax, f->inst, f->inst_sorted));
+    UDX_TRY(clist_sort_aos(s, &f->cl, nmax, f->inst, f->inst_sorted));
     const int nc = f->cl.box.ncells();
     hipLaunchKernelGGL(k_gather_int2, dim3(ceil_div(nmax, 256)), dim3(256), 0, s, nmax, f->cl.starts + nc,
                        f->cl.order, f->meta, f->meta_sorted);

@@ -89,7 +89,6 @@ extern "C" int udx_clist_build_noalloc(udx_ctx *ctx, int Lx, int Ly, int Lz, int
     c.order = order;
     c.scan_tmp = base + NA_SCAN;
     hipStream_t s = ctx->stream;
-    UDX_TRY(clist_sort_aos(s, &c, n, pp));
-    if (ppout) UDX_TRY(gather_aos(s, &c, n, pp, ppout));
+    UDX_TRY(clist_sort_aos(s, &c, n, pp, ppout));
     return UDX_OK;
 }

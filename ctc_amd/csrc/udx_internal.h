@@ -94,28 +94,24 @@ struct ClistBufs {
 constexpr int SOLVENT_SUB = 4;
 int clist_alloc(ClistBufs *c, const Box &b, int maxp, int sub = 1);
 void clist_free(ClistBufs *c);
-// pos4 (input, n particles): counting sort into cell order; order[] and
-// starts[] filled; the number kept is starts[ncells] on the device
-int clist_sort(hipStream_t s, ClistBufs *c, int n, const float4 *pos4);
-int clist_sort_aos(hipStream_t s, ClistBufs *c, int n, const float *pp);
-// the two halves of a sort for callers that fill bcounts[] and cellslot[]
-// themselves: zero the slab counts; scan, scatter, the stable in-slab order
-// and the cell tables
+// pp (AoS, n particles): counting sort into cell order; order[] and starts[]
+// filled, the particles copied to ppout in that order (unless null); the
+// number kept is starts[ncells] on the device
+int clist_sort_aos(hipStream_t s, ClistBufs *c, int n, const float *pp, float *ppout);
+// the two halves of a sort of float4 streams, for callers that may fill
+// bcounts[] and cellslot[] themselves (zero the slab counts first): the
+// counts; then scan, scatter, the stable in-slab order with the particles
+// copied to it (order[] itself is scratch) and the cell tables
 int clist_clear(hipStream_t s, ClistBufs *c);
-int clist_finish(hipStream_t s, ClistBufs *c, int n);
-// the counting half alone (clist_finish completes the sort)
 int clist_count_only(hipStream_t s, ClistBufs *c, int n, const float4 *pos4);
-// out[k] = in[order[k]] for k < starts[ncells]; n bounds the launch
-int gather_f4(hipStream_t s, const ClistBufs *c, int n, const float4 *pin, const float4 *vin,
-              float4 *pout, float4 *vout);
-int gather_aos(hipStream_t s, const ClistBufs *c, int n, const float *pin, float *pout);
+int clist_finish_f4(hipStream_t s, ClistBufs *c, int n, const float4 *pin, const float4 *vin, float4 *pout,
+                    float4 *vout);
 
 // ------------------------------------------------------------------ forces
 struct FragTables {
-    int *cnt;        // cell counts of the 26 fragments, concatenated (one 0 after each)
-    int *fss;        // exclusive scan of cnt: fragment f's offsets are fss[off[f] + h] - fss[off[f]]
-    int *scan_tmp;
-    int off[27];     // start of each fragment in cnt
+    int *fss;        // packed-list offsets of the 26 fragments' cells: fragment f's are fss[off[f] + h]
+    int *cnt;        // the cells' counts, for boxes with large faces (else null)
+    int off[27];     // start of each fragment in fss
     int size;
 };
 struct FragOff {
@@ -123,8 +119,21 @@ struct FragOff {
 };
 int frag_alloc(FragTables *t, const Box &b);
 void frag_free(FragTables *t);
+// the step's seeds read on the device (a captured step): cur = the nseed
+// seeds of step *step in the table, then *step advanced
+struct StepSeeds {
+    const float *table = nullptr;
+    int *step = nullptr;
+    float *cur = nullptr;
+    int nseed = 0;
+};
 // ecount (optional): a box's edge list counter, cleared here for the step
-int frag_build(hipStream_t s, const FragTables *t, const Box &b, const int *starts, int *ecount = nullptr);
+int frag_build(hipStream_t s, const FragTables *t, const Box &b, const int *starts, int *ecount = nullptr,
+               const StepSeeds &seeds = StepSeeds{});
+// the same for the boxes of a batch, laid end to end: fragment tables at
+// fbase + foff (27 per box), cells from coff; seeds of every box
+int frag_build_batch(hipStream_t s, int nbox, const int *fbase, const int *foff, const int *coff, const int4 *boxL,
+                     const int *starts, int *fss, int *ecount, const float *table, const int *step, float *seeds);
 
 // entries a gather may read past a lane's last candidate (values unused): the
 // position streams it reads have this many more than their particles

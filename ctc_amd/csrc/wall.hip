@@ -609,8 +609,7 @@ int wall_build_frozen(hipStream_t s, WallSet *w, const SdfField *q, int nw, floa
     float *sorted = nullptr;
     if (!st) st = dev_alloc(&sorted, 6L * (ntot > 0 ? ntot : 1));
     if (!st) st = dev_alloc(&w->pos, (size_t)ntot + POS_PAD);
-    if (!st) st = clist_sort_aos(s, &w->cl, ntot, all);
-    if (!st) st = gather_aos(s, &w->cl, ntot, all, sorted);
+    if (!st) st = clist_sort_aos(s, &w->cl, ntot, all, sorted);
     if (!st && ntot > 0) {
         hipLaunchKernelGGL(k_aos_pos4, dim3(ceil_div(ntot, 256)), dim3(256), 0, s, ntot, sorted, w->pos);
         if (hipGetLastError() != hipSuccess) st = UDX_EHIP;
