@@ -98,14 +98,19 @@ __global__ __launch_bounds__(256) void k_sdf_resample(const float *D, Grid g, in
     for (int c = 0; c < 3; c++) anchor[c] = (int)__builtin_floorf(r[c]);
     for (int c = 0; c < 3; c++)
         for (int i = 0; i < 4; i++) w[c][i] = spl(r[c] - (float)(anchor[c] - 1 + i) + 2);
+    // the margin of a box thinner than it reaches past the field's first copy
+    auto wrap = [](int i, int n) {
+        i %= n;
+        return i < 0 ? i + n : i;
+    };
     float tmp[4][4], partial[4];
     for (int sz = 0; sz < 4; sz++)
         for (int sy = 0; sy < 4; sy++) {
             float s = 0;
-            const int gz = (sz - 1 + anchor[2] + g.N[2]) % g.N[2];
-            const int gy = (sy - 1 + anchor[1] + g.N[1]) % g.N[1];
+            const int gz = wrap(sz - 1 + anchor[2], g.N[2]);
+            const int gy = wrap(sy - 1 + anchor[1], g.N[1]);
             for (int sx = 0; sx < 4; sx++) {
-                const int gx = (sx - 1 + anchor[0] + g.N[0]) % g.N[0];
+                const int gx = wrap(sx - 1 + anchor[0], g.N[0]);
                 s += w[0][sx] * D[gx + g.N[0] * (gy + (long)g.N[1] * gz)];
             }
             tmp[sz][sy] = s;

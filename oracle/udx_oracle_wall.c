@@ -90,7 +90,7 @@ static float spl_get(const int N[3], const float *D, const float r[3]) {
             s = 0;
             for (int sx = 0; sx < 4; sx++) {
                 int l[3] = {sx, sy, sz};
-                for (int c = 0; c < 3; c++) g[c] = (l[c] - 1 + anchor[c] + N[c]) % N[c];
+                for (int c = 0; c < 3; c++) g[c] = ((l[c] - 1 + anchor[c]) % N[c] + N[c]) % N[c];
                 s += w[0][sx] * D[g[0] + N[0] * (g[1] + N[1] * g[2])];
             }
             tmp[sz][sy] = s;
