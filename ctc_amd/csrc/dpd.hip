@@ -1848,8 +1848,9 @@ __device__ __forceinline__ void frag_table(int n, const Count &count, int *fss) 
 
 // Faces of more than FRAG_FACE cells are counted by a launch of their own: the
 // cells of an x face lie a row apart, a cache line each, more than one CU
-// fetches in good time (96^2 faces: 44 us for the one launch).
-constexpr int FRAG_FACE = 4096;
+// fetches in good time (one launch: 4.8 us at 40 x 37 cells, 16 at 64 x 64, 44
+// at 96 x 96; two: 13 at 96 x 96).
+constexpr int FRAG_FACE = 2048;
 __global__ __launch_bounds__(256) void k_frag_counts(const int *starts, int Lx, int Ly, int Lz, FragOff fo, int *cnt) {
     const int g = blockIdx.x * blockDim.x + threadIdx.x;
     if (g >= fo.off[26]) return;

@@ -276,12 +276,26 @@ struct SdfView {
     float cheap_threshold;
 };
 
-// point fetch with wrap addressing (src/wall/sdf/tex3d/imp/main.h:12-29)
-__device__ __forceinline__ float sdf_fetch(const SdfView &v, int i, int j, int k) {
-    i %= v.T[0]; if (i < 0) i += v.T[0];
-    j %= v.T[1]; if (j < 0) j += v.T[1];
-    k %= v.T[2]; if (k < 0) k += v.T[2];
+// wrap addressing of one texel index (src/wall/sdf/tex3d/imp/main.h:12-29).
+// The texture covers the box and its margin, so a particle's indices are
+// inside it: the remainder, about forty instructions each, is taken only by
+// waves with an index outside.
+__device__ __forceinline__ int sdf_wrap(int i, int T) {
+    if ((unsigned)i >= (unsigned)T) {
+        i %= T;
+        if (i < 0) i += T;
+    }
+    return i;
+}
+
+// texel at wrapped indices
+__device__ __forceinline__ float sdf_texel(const SdfView &v, int i, int j, int k) {
     return v.tex[i + v.T[0] * ((long)j + (long)v.T[1] * k)];
+}
+
+// point fetch
+__device__ __forceinline__ float sdf_fetch(const SdfView &v, int i, int j, int k) {
+    return sdf_texel(v, sdf_wrap(i, v.T[0]), sdf_wrap(j, v.T[1]), sdf_wrap(k, v.T[2]));
 }
 
 __device__ __forceinline__ void sdf_tex(const SdfView &v, float x, float y, float z, float t[3]) {
@@ -293,16 +307,18 @@ __device__ __forceinline__ void sdf_tex(const SdfView &v, float x, float y, floa
 // trilinear interpolation between texel centres (src/wall/sdf/dev.h:79-112)
 __device__ __forceinline__ float sdf_eval(const SdfView &v, float x, float y, float z) {
     float t[3], l[3];
-    int c0[3];
+    int a[3], b[3];   // the texels on both sides, per axis
     sdf_tex(v, x, y, z, t);
     for (int c = 0; c < 3; c++) {
-        c0[c] = (int)t[c];
-        l[c] = t[c] - (float)c0[c];
+        const int c0 = (int)t[c];
+        l[c] = t[c] - (float)c0;
+        a[c] = sdf_wrap(c0, v.T[c]);
+        b[c] = sdf_wrap(c0 + 1, v.T[c]);
     }
-    const float s000 = sdf_fetch(v, c0[0], c0[1], c0[2]), s001 = sdf_fetch(v, c0[0] + 1, c0[1], c0[2]);
-    const float s010 = sdf_fetch(v, c0[0], c0[1] + 1, c0[2]), s011 = sdf_fetch(v, c0[0] + 1, c0[1] + 1, c0[2]);
-    const float s100 = sdf_fetch(v, c0[0], c0[1], c0[2] + 1), s101 = sdf_fetch(v, c0[0] + 1, c0[1], c0[2] + 1);
-    const float s110 = sdf_fetch(v, c0[0], c0[1] + 1, c0[2] + 1), s111 = sdf_fetch(v, c0[0] + 1, c0[1] + 1, c0[2] + 1);
+    const float s000 = sdf_texel(v, a[0], a[1], a[2]), s001 = sdf_texel(v, b[0], a[1], a[2]);
+    const float s010 = sdf_texel(v, a[0], b[1], a[2]), s011 = sdf_texel(v, b[0], b[1], a[2]);
+    const float s100 = sdf_texel(v, a[0], a[1], b[2]), s101 = sdf_texel(v, b[0], a[1], b[2]);
+    const float s110 = sdf_texel(v, a[0], b[1], b[2]), s111 = sdf_texel(v, b[0], b[1], b[2]);
     // A (1 - p) + p B with the first product fused into the sum
     auto wav = [](float A, float B, float p) { return __builtin_fmaf(A, 1 - p, p * B); };
     const float s00x = wav(s000, s001, l[0]), s01x = wav(s010, s011, l[0]);
@@ -315,11 +331,15 @@ __device__ __forceinline__ float sdf_eval(const SdfView &v, float x, float y, fl
 __device__ __forceinline__ void sdf_grad(const SdfView &v, float x, float y, float z, float g[3]) {
     float t[3];
     sdf_tex(v, x, y, z, t);
-    const int i = (int)t[0], j = (int)t[1], k = (int)t[2];
-    const float s0 = sdf_fetch(v, i, j, k);
-    g[0] = v.s[0] * (sdf_fetch(v, i + 1, j, k) - s0);
-    g[1] = v.s[1] * (sdf_fetch(v, i, j + 1, k) - s0);
-    g[2] = v.s[2] * (sdf_fetch(v, i, j, k + 1) - s0);
+    int i[3], u[3];
+    for (int c = 0; c < 3; c++) {
+        i[c] = sdf_wrap((int)t[c], v.T[c]);
+        u[c] = sdf_wrap((int)t[c] + 1, v.T[c]);
+    }
+    const float s0 = sdf_texel(v, i[0], i[1], i[2]);
+    g[0] = v.s[0] * (sdf_texel(v, u[0], i[1], i[2]) - s0);
+    g[1] = v.s[1] * (sdf_texel(v, i[0], u[1], i[2]) - s0);
+    g[2] = v.s[2] * (sdf_texel(v, i[0], i[1], u[2]) - s0);
 }
 
 __device__ __forceinline__ void sdf_ugrad(const SdfView &v, float x, float y, float z, float g[3]) {
