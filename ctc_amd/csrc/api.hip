@@ -743,7 +743,8 @@ static int flu_step(udx_flu *f, const float *seeds_dev, const float *fsi_seeds, 
             if (m.wall_lambda > 0) UDX_TRY(wall_repulse_aos(s, sdf, m.wall_lambda, nvtx, m.pp, m.fo));
         }
         // FSI: +f on the vertices, -f on the solvent (src/sim/objinter/imp/main.h:42-91)
-        UDX_TRY(fsi_forces(s, fsi_bufs(m.fsi), f->n, f->pos[b], f->vel[b], f->cl.starts, nvtx, m.pp, m.fp, fsi_seeds,
+        UDX_TRY(fsi_forces(s, fsi_bufs(m.fsi), f->n, f->pos[b], f->vel[b], f->cl.starts, f->cl.bstarts,
+                           f->cl.sub, nvtx, m.pp, m.fp, fsi_seeds,
                            m.fo, (float *)f->ff, 4, fsi_pairs_dev(m.fsi), f->conf.mode == UDX_MODE_EXACT));
         // contact (forces_cnt, cnt_halo: src/sim/objinter/imp/main.h:22-26,79)
         if (m.cnt) {

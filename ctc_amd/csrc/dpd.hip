@@ -82,22 +82,6 @@ struct DpdK {
 // candidate loops would also wait for the outstanding particle loads.  The
 // scalars are copied so that the loops do not read them from the table again
 // (a read inside a conditional block cannot be hoisted out of the loop).
-#define UDX_GLOBAL __attribute__((address_space(1)))
-typedef float f4v __attribute__((ext_vector_type(4)));
-typedef float f3v __attribute__((ext_vector_type(3)));   // 16 B in memory; loads read 12
-
-template <class T>
-__device__ __forceinline__ UDX_GLOBAL T *gptr(T *p) {
-    return (UDX_GLOBAL T *)p;
-}
-
-// x, y, z of the entry at a byte offset, plus K entries folded into the load.
-// The 32-bit offset (indices stay below 2^27) goes into the load beside the
-// base; a signed index takes five more instructions per particle to widen.
-__device__ __forceinline__ f3v pos_at(const UDX_GLOBAL f4v *p, unsigned byte, int k) {
-    return *(const UDX_GLOBAL f3v *)((const UDX_GLOBAL char *)p + (size_t)byte + 16 * k);
-}
-
 struct DpdP {
     const UDX_GLOBAL f4v *pos, *vel;
     const UDX_GLOBAL int *starts, *fss, *bstarts;
@@ -240,75 +224,6 @@ __device__ __forceinline__ PairIn pair_in_wrapped(const DpdP &P, unsigned ent, i
     pair_kin(o, ax, ay, az, vi, pj, vj);
     o.x = P.seeds[frag_d2i(wx, wy, wz)] - low_discrepancy((float)(u & 0x3FF), (float)u, (float)(v & 0x3FF), (float)v);
     return o;
-}
-
-// v summed over the lanes up to this one
-__device__ __forceinline__ int wave_scan_add(int v) {
-    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);   // row_shr:1
-    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);   // row_bcast:15
-    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);   // row_bcast:31
-    return v;
-}
-
-// smallest and largest value over the wave's lanes
-__device__ __forceinline__ int wave_min(int v) {
-    v = min(v, __builtin_amdgcn_update_dpp(0x7fffffff, v, 0x111, 0xf, 0xf, false));
-    v = min(v, __builtin_amdgcn_update_dpp(0x7fffffff, v, 0x112, 0xf, 0xf, false));
-    v = min(v, __builtin_amdgcn_update_dpp(0x7fffffff, v, 0x114, 0xf, 0xf, false));
-    v = min(v, __builtin_amdgcn_update_dpp(0x7fffffff, v, 0x118, 0xf, 0xf, false));
-    v = min(v, __builtin_amdgcn_update_dpp(0x7fffffff, v, 0x142, 0xa, 0xf, false));
-    v = min(v, __builtin_amdgcn_update_dpp(0x7fffffff, v, 0x143, 0xc, 0xf, false));
-    return __builtin_amdgcn_readlane(v, 63);
-}
-__device__ __forceinline__ int wave_max(int v) { return -wave_min(-v); }
-
-// Candidate window along x.  With x-slab starts a row run [x0, x1] of cells
-// (wrap wx) is cut to the slabs that can hold a particle within the cutoff:
-// a candidate at y-z distance >= d from the particle has |dx| < sqrt(1 - d^2).
-// The bound is conservative for the float pair test: the y-z gaps g are
-// lowered and the half-width raised by WIN_MARGIN (above the rounding of
-// the particle's periodic shift for boxes up to 2048 cells) and 1 + 1e-5
-// stands for the cutoff, so every candidate the test would accept lies in
-// the window.  hw < 0: no particle of the row is within the cutoff.
-constexpr float WIN_MARGIN = 1.0f / 4096.0f;
-
-__device__ __forceinline__ float row_halfwidth(int dy, int dz, float fy, float fz) {
-    float gy = dy == 0 ? 0.f : (dy < 0 ? fy : 1.f - fy);
-    float gz = dz == 0 ? 0.f : (dz < 0 ? fz : 1.f - fz);
-    gy = fmaxf(gy - WIN_MARGIN, 0.f);
-    gz = fmaxf(gz - WIN_MARGIN, 0.f);
-    const float w2 = 1.00001f - gy * gy - gz * gz;
-    return w2 < 0.f ? -1.f : __builtin_amdgcn_sqrtf(w2) + WIN_MARGIN;
-}
-
-// candidates of the run [x0, x1] of the row starting at cell `base`, for a
-// particle in column c of the run's frame (its own column less the wrap times
-// the box side), fx into its cell: index range [*j, *j + *n).  The window is
-// counted in slabs from the particle's cell, so floats hold it exactly enough
-// for the margin (slabs counted from the box edge need doubles, three times
-// the issue cycles).
-__device__ __forceinline__ void run_range(const DpdP &P, int base, int x0, int x1, int c, float fx, float hw, int *j,
-                                          int *n) {
-    const UDX_GLOBAL int *st = P.starts;
-    int lo = base + x0, hi = base + x1;
-    if (P.bstarts) {
-        const int S = P.sub;
-        st = P.bstarts;
-        lo = max(c * S + (int)__builtin_floorf((fx - hw) * (float)S), x0 * S);
-        hi = min(c * S + (int)__builtin_floorf((fx + hw) * (float)S), x1 * S + S - 1);
-        if (!(hw >= 0.f) || lo > hi) {
-            *j = 0;
-            *n = 0;
-            return;
-        }
-        lo += base * S;
-        hi += base * S;
-    }
-    *j = st[lo];
-    *n = st[hi + 1] - *j;
 }
 
 template <bool B>
@@ -618,7 +533,7 @@ __device__ __forceinline__ void dpd_block(const DpdK &A, int first) {
         int j0 = 0, n0 = 0;
         if (active && yy >= 0 && yy < Ly && zz >= 0 && zz < Lz) {
             const int x0 = cx > 0 ? cx - 1 : 0, x1 = cx + 1 < Lx ? cx + 1 : Lx - 1;
-            run_range(P, Lx * (yy + Ly * zz), x0, x1, cx, rx, row_halfwidth(dy, dz, ry, rz), &j0, &n0);
+            run_range(P.starts, P.bstarts, P.sub, Lx * (yy + Ly * zz), x0, x1, cx, rx, row_halfwidth(dy, dz, ry, rz), &j0, &n0);
         }
         // the union of the wave's candidate ranges of this row
         const int lo = wave_min(n0 > 0 ? j0 : 0x7fffffff), hi = wave_max(n0 > 0 ? j0 + n0 : 0);
@@ -772,11 +687,11 @@ __device__ __forceinline__ void dpd_block(const DpdK &A, int first) {
                 const float hw = row_halfwidth(dy, dz, ry, rz);
                 const int base = Lx * (yy + Ly * zz);
                 if (xrun(0, cx, Lx, &x0, &x1, &wx0) && (yzwrap || wx0 != 0)) {
-                    run_range(P, base, x0, x1, cx - wx0 * Lx, rx, hw, &j0, &n0);
+                    run_range(P.starts, P.bstarts, P.sub, base, x0, x1, cx - wx0 * Lx, rx, hw, &j0, &n0);
                     if (n0 > 0) runtab(wx0, x0, &aid0, &b0, &m0);
                 }
                 if (xrun(1, cx, Lx, &x0, &x1, &wx1) && (yzwrap || wx1 != 0)) {
-                    run_range(P, base, x0, x1, cx - wx1 * Lx, rx, hw, &j1, &n1);
+                    run_range(P.starts, P.bstarts, P.sub, base, x0, x1, cx - wx1 * Lx, rx, hw, &j1, &n1);
                     if (n1 > 0) runtab(wx1, x0, &aid1, &b1, &m1);
                 }
             }
@@ -1002,46 +917,6 @@ constexpr int CO_WAVES = 9, CO_THREADS = 64 * CO_WAVES;
 constexpr int CO_STAGE = 128;               // candidates a wave stages in LDS
 constexpr int CO_CAP = 3072;                // pair slots of a block (density 10 has about 2600)
 constexpr unsigned CO_DENSE = 0xFFu;        // a row with more than 64 candidates in a run
-
-// hits of up to 64 candidates as bits, candidate k at bit 31 - (k mod 32) of
-// word k / 32: the sign of r2 - 1, shifted in from the right.  at(k) reads the
-// lane's candidate k, for k up to seven past the last one.
-struct Mask64 {
-    unsigned w[2];
-};
-template <class At>
-__device__ __forceinline__ Mask64 test64(int n, float ax, float ay, float az, At at) {
-    Mask64 m{{0u, 0u}};
-#pragma unroll
-    for (int c = 0; c < 2; c++) {
-        if (!wave_any(n > 32 * c)) break;
-        unsigned b = 0;
-        int sh = 32;
-        f3v q[4], nx[4];
-#pragma unroll
-        for (int u = 0; u < 4; u++) q[u] = at(32 * c + u);
-#pragma unroll
-        for (int g = 0; g < 8; g++) {
-            if (g && !wave_any(n > 32 * c + 4 * g)) break;
-            if (g < 7)
-#pragma unroll
-                for (int u = 0; u < 4; u++) nx[u] = at(32 * c + 4 * (g + 1) + u);
-#pragma unroll
-            for (int u = 0; u < 4; u++) {
-                const float dx = ax - q[u].x, dy = ay - q[u].y, dz = az - q[u].z;
-                const float r2 = __builtin_fmaf(dz, dz, __builtin_fmaf(dx, dx, dy * dy));
-                b = __builtin_amdgcn_alignbit(b, __float_as_uint(r2 - 1.0f), 31);
-            }
-            sh -= 4;
-#pragma unroll
-            for (int u = 0; u < 4; u++) q[u] = nx[u];
-        }
-        b <<= sh & 31;
-        const int left = n - 32 * c;
-        m.w[c] = left >= 32 ? b : (left > 0 ? b & ~(0xFFFFFFFFu >> left) : 0u);
-    }
-    return m;
-}
 
 struct CoopLds {
     float4 hp[64], hv[64];
@@ -1341,7 +1216,7 @@ __device__ __forceinline__ void coop_block(const DpdK &A, int first, CoopLds &S)
         }
         auto range = [&](Run &r) {
             r.ax = pi.x - (float)(r.wx * Lx);
-            if (r.on) run_range(P, base, r.x0, r.x1, cx - r.wx * Lx, rx, hw, &r.j, &r.n);
+            if (r.on) run_range(P.starts, P.bstarts, P.sub, base, r.x0, r.x1, cx - r.wx * Lx, rx, hw, &r.j, &r.n);
             r.on = r.n > 0;
             r.j = r.on ? r.j - i0 : 0;
         };
@@ -1586,7 +1461,7 @@ __device__ __forceinline__ void dpd_half_block(const DpdK &A, int first, HsWave 
         if (active && yy >= 0 && yy < Ly && zz >= 0) {
             const int x0 = cx > 0 ? cx - 1 : 0;
             const int x1 = row == 4 ? cx : (cx + 1 < Lx ? cx + 1 : Lx - 1);
-            run_range(P, Lx * (yy + Ly * zz), x0, x1, cx, rx, row_halfwidth(dy, dz, ry, rz), &j0, &n0);
+            run_range(P.starts, P.bstarts, P.sub, Lx * (yy + Ly * zz), x0, x1, cx, rx, row_halfwidth(dy, dz, ry, rz), &j0, &n0);
             if (row == 4) n0 = max(0, min(n0, i - j0));   // own row: lower indices only
         }
         const int lo = wave_min(n0 > 0 ? j0 : 0x7fffffff), hi = wave_max(n0 > 0 ? j0 + n0 : 0);
@@ -1692,9 +1567,9 @@ __device__ __forceinline__ void dpd_half_block(const DpdK &A, int first, HsWave 
                 const float hw = row_halfwidth(dy, dz, ry, rz);
                 const int base = Lx * (yy + Ly * zz);
                 if (xrun(0, cx, Lx, &x0, &x1, &wx0) && (yzwrap || wx0 != 0))
-                    run_range(P, base, x0, x1, cx - wx0 * Lx, rx, hw, &j0, &n0);
+                    run_range(P.starts, P.bstarts, P.sub, base, x0, x1, cx - wx0 * Lx, rx, hw, &j0, &n0);
                 if (xrun(1, cx, Lx, &x0, &x1, &wx1) && (yzwrap || wx1 != 0))
-                    run_range(P, base, x0, x1, cx - wx1 * Lx, rx, hw, &j1, &n1);
+                    run_range(P.starts, P.bstarts, P.sub, base, x0, x1, cx - wx1 * Lx, rx, hw, &j1, &n1);
             }
             const float ay = pi.y - (float)(wy * Ly), az = pi.z - (float)(wz * Lz);
             const float ax0 = pi.x - (float)(wx0 * Lx), ax1 = pi.x - (float)(wx1 * Lx);

@@ -92,7 +92,8 @@ __global__ __launch_bounds__(256) void k_fsi_instances(int no, const float *opp,
 struct FsiK {
     int Lx, Ly, Lz;
     const float4 *spos, *svel;
-    const int *starts;
+    const int *starts, *bstarts;   // cell starts, x-slab starts (sub per cell) or null
+    int sub;
     DpdPar par;
     const float *seeds;      // device: [bulk, halo]
 };
@@ -103,159 +104,158 @@ struct FsiK {
 // one candidate in six passes and every lane of the wave would wait for the
 // body at nearly every candidate.  The queues keep candidate order, so the
 // sums are the same as a sequential walk.
-constexpr int FQ_V = 16, FQ_S = 16;   // ring entries per lane: instance side, solvent side
+constexpr int FQ_S = 16;   // ring entries per lane
 constexpr int FSI_DRAIN_STEPS = 2;
 constexpr int FSI_SCAP = 160;         // staged instances per wave and row (solvent side)
-constexpr int FSI_VCAP = 160;         // staged solvent particles per wave and row (instance side)
 struct FsiIn {
     float dx, dy, dz, r2, dvx, dvy, dvz, x;
     bool pair;
 };
 
-// Vertex side, one thread per instance (the vertex or one of its images)
-// in cell order of the instance grid, so the lanes of a wave read the same
-// solvent cells: the instance's sum over its clipped block, z planes 0..2,
-// rows y - 1..y + 1, solvent in cell order (src/fsi/dev/map/bulk.h), written
-// to sinst at the instance's own index.  k_fsi_vertex_sum then adds, per
-// vertex, its own sum and its images' sums in halo-list order.
+// Vertex side: seven instances (the vertex or one of its images) to a wave, in
+// cell order of the instance grid, nine lanes each, one per row of its block
+// (z planes 0..2, rows y - 1..y + 1: src/fsi/dev/map/bulk.h).  The lane tests its
+// row's candidates; lanes are in the order of the sums, so a scan of their
+// hits places every pair in one list of the wave, which all lanes evaluate, and
+// a lane per instance and force component adds its pairs in order.  The sum is
+// written to sinst at the instance's own index.  Bound by issue and the per-lane
+// loads when there are many, by one chain of about 20 thousand cycles when
+// there are few: a lane per instance was a chain of 42 pairs behind the
+// candidates of all nine rows (5184 vertices at density 10: 78 -> 12 us;
+// 329 thousand: 204 -> 164 us, whose rows are now cut to x slabs too).
+constexpr int FI_HOMES = 7, FI_WAVES = 4, FI_CAP = 448;
 template <int WR, bool EXACT>
-__global__ __launch_bounds__(FSI_THREADS) void k_fsi_instance(FsiK K, const int *n_dev, const float *inst,
-                                                              const int2 *meta, const int *order, float *sinst,
-                                                              unsigned long long *pairs) {
-    __shared__ unsigned q[FQ_V * FSI_THREADS];
-    __shared__ float4 vstage[FSI_THREADS / 64][FSI_VCAP];
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    const bool active = t < *n_dev;
-    float4 *const sv = vstage[threadIdx.x >> 6];
-    const float *p = inst + 6 * (long)(active ? t : 0);
-    const float rx = p[0], ry = p[1], rz = p[2], ux = p[3], uy = p[4], uz = p[5];
-    const int2 m = active ? meta[t] : make_int2(0, 0);
-    const unsigned lid = (unsigned)m.x;
-    const float seed = m.y ? K.seeds[1] : K.seeds[0];
-    float sx = 0.f, sy = 0.f, sz = 0.f;
-    int fill = 0, head = 0, np = 0;
-    unsigned *ql = q + threadIdx.x;
-    auto ring = [&](int k) {
-        const int r = head + k;
-        return r >= FQ_V ? r - FQ_V : r;
+__global__ __launch_bounds__(64 * FI_WAVES) void k_fsi_instance(FsiK K, const int *n_dev, const float *inst,
+                                                                const int2 *meta, const int *order, float *sinst,
+                                                                unsigned long long *pairs) {
+    struct Wave {
+        float4 hp[FI_HOMES], hv[FI_HOMES];   // position and noise index; velocity and seed
+        unsigned item[3][FI_CAP];            // a pair: home << 27 | solvent particle; then its force
     };
-    auto in_of = [&](unsigned b) {
-        FsiIn o;
-        const float4 pb = K.spos[b], vb = K.svel[b];
-        o.dx = rx - pb.x;
-        o.dy = ry - pb.y;
-        o.dz = rz - pb.z;
-        o.r2 = __builtin_fmaf(o.dz, o.dz, __builtin_fmaf(o.dx, o.dx, o.dy * o.dy));
-        o.dvx = ux - vb.x;
-        o.dvy = uy - vb.y;
-        o.dvz = uz - vb.z;
-        // mean0var1uu(seed, lid, b) before the logistic map (src/math/rnd/dev.h:65-72)
-        o.x = seed - low_discrepancy((float)(lid & 0x3FFu), (float)lid, (float)(b & 0x3FFu), (float)b);
-        o.pair = true;
-        return o;
-    };
-    auto drain_step = [&]() {
-        const bool va = fill > 0, vb = fill > 1;
-        const unsigned ea = va ? ql[ring(0) * FSI_THREADS] : 0u;     // solvent 0 exists when anything is queued
-        const unsigned eb = vb ? ql[ring(1) * FSI_THREADS] : ea;
-        const FsiIn a = in_of(ea), b = in_of(eb);
-        float xa = a.x, xb = b.x;
-        logistic18x2(&xa, &xb);
-        const float3 fa = dpd_pair<WR, EXACT>(K.par, a.dx, a.dy, a.dz, a.r2, a.dvx, a.dvy, a.dvz, xa * R_SQRT2);
-        const float3 fb = dpd_pair<WR, EXACT>(K.par, b.dx, b.dy, b.dz, b.r2, b.dvx, b.dvy, b.dvz, xb * R_SQRT2);
-        if (va) {
-            sx += fa.x;
-            sy += fa.y;
-            sz += fa.z;
-        }
-        if (vb) {
-            sx += fb.x;
-            sy += fb.y;
-            sz += fb.z;
-        }
-        const int took = fill < 2 ? fill : 2;
-        np += took;
-        head = ring(took);
-        fill -= took;
-    };
-    const int xc = K.Lx / 2 + (int)__builtin_floorf(rx);
-    const int yc = K.Ly / 2 + (int)__builtin_floorf(ry);
-    const int zc = K.Lz / 2 + (int)__builtin_floorf(rz);
-    const bool xok = active && !(xc - 1 >= K.Lx || xc + 2 <= 0);
-    const int xs = xc - 1 > 0 ? xc - 1 : 0, xe = xc + 2 < K.Lx ? xc + 2 : K.Lx;
-    for (int row = 0; row < 9; row++) {
-        const int z = zc - 1 + row / 3, y = yc - 1 + row % 3;
-        int b0 = 0, len = 0;
-        if (xok && z >= 0 && z < K.Lz && y >= 0 && y < K.Ly) {
-            const int cid = xs + K.Lx * (y + K.Ly * z);
-            b0 = K.starts[cid];
-            len = K.starts[cid + (xe - xs)] - b0;
-        }
-        // the lanes are consecutive instances in cell order: the union of
-        // their solvent runs of this row is usually one small range, staged
-        // in LDS with coalesced loads (one round trip instead of one per four
-        // candidates); the candidate order is the same either way
-        int lo = len > 0 ? b0 : 0x7fffffff, hi = len > 0 ? b0 + len : 0;
-#pragma unroll
-        for (int d = 32; d >= 1; d >>= 1) {
-            lo = min(lo, __shfl_xor(lo, d, 64));
-            hi = max(hi, __shfl_xor(hi, d, 64));
-        }
-        if (hi <= lo) continue;
-        if (hi - lo <= FSI_VCAP) {
+    __shared__ Wave lds[FI_WAVES];
+    __shared__ int count[FI_WAVES];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    Wave &S = lds[w];
+    const int n = *n_dev;
+    const int first = (blockIdx.x * FI_WAVES + w) * FI_HOMES;
+    if (blockIdx.x * FI_WAVES * FI_HOMES >= n) return;
+    const UDX_GLOBAL f4v *const spos = (const UDX_GLOBAL f4v *)K.spos, *const svel = (const UDX_GLOBAL f4v *)K.svel;
+    const int h = lane / 9, row = lane % 9;
+    const bool active = h < FI_HOMES && first + h < n;
+    const float *p = inst + 6 * (long)(active ? first + h : 0);
+    const float rx = p[0], ry = p[1], rz = p[2];
+    if (active && row == 0) {
+        const int2 m = meta[first + h];
+        S.hp[h] = make_float4(rx, ry, rz, __int_as_float(m.x));
+        S.hv[h] = make_float4(p[3], p[4], p[5], m.y ? K.seeds[1] : K.seeds[0]);
+    }
+    int j = 0, m = 0;
+    {
+        const float flx = __builtin_floorf(rx), fly = __builtin_floorf(ry), flz = __builtin_floorf(rz);
+        const int xc = K.Lx / 2 + (int)flx, yc = K.Ly / 2 + (int)fly, zc = K.Lz / 2 + (int)flz;
+        const int dz = row / 3 - 1, dy = row % 3 - 1, z = zc + dz, y = yc + dy;
+        const int xs = xc - 1 > 0 ? xc - 1 : 0, xe = xc + 2 < K.Lx ? xc + 2 : K.Lx;
+        const float hw = row_halfwidth(dy, dz, ry - fly, rz - flz);
+        if (active && xc - 1 < K.Lx && xc + 2 > 0 && z >= 0 && z < K.Lz && y >= 0 && y < K.Ly && hw >= 0.f)
+            run_range((const UDX_GLOBAL int *)K.starts, (const UDX_GLOBAL int *)K.bstarts, K.sub,
+                      K.Lx * (y + K.Ly * z), xs, xe - 1, xc, rx - flx, hw, &j, &m);
+    }
+    float acc = 0.f;   // lane c FI_HOMES + g: component c of instance first + g
+    int np = 0;
+    // sel < 0: every row, its first 64 candidates; else (a row has more) one row at a time
+    int sel = wave_any(m > 64) ? 0 : -1, skip = 0;
+    for (;;) {
+        const int nc = sel < 0 || sel == row ? m - skip : 0;
+        const unsigned byte = (unsigned)(nc > 0 ? j + skip : 0) * 16u;
+        const Mask64 mk = test64(nc, rx, ry, rz, [&](int k) { return pos_at(spos, byte, k); });
+        const int end = wave_scan_add(__popc(mk.w[0]) + __popc(mk.w[1]));
+        const int off = end - (__popc(mk.w[0]) + __popc(mk.w[1]));
+        const int T = __builtin_amdgcn_readlane(end, 63);
+        np += T;
+        const int g = lane % FI_HOMES, comp = lane / FI_HOMES;   // the sums' lanes: comp < 3
+        const int g0 = __shfl(off, 9 * g, 64), g1 = __shfl(end, 9 * g + 8, 64);
+        for (int c0 = 0; c0 < T; c0 += FI_CAP) {
             __builtin_amdgcn_wave_barrier();
-            for (int k = threadIdx.x & 63; k < hi - lo; k += 64) sv[k] = K.spos[lo + k];
-            __builtin_amdgcn_wave_barrier();
-            const int o = len > 0 ? b0 - lo : 0;
-            for (int c = 0; wave_any(c < len); c += 4) {
-                if (wave_any(fill + 4 > FQ_V))
-#pragma unroll 1
-                    for (int k = 0; k < FSI_DRAIN_STEPS; k++) drain_step();
+            int at = off - c0;
 #pragma unroll
-                for (int u = 0; u < 4; u++) {
-                    const int k = o + c + u < FSI_VCAP ? o + c + u : 0;
-                    const float4 pb = c + u < len ? sv[k] : make_float4(1e30f, 1e30f, 1e30f, 0.f);
-                    const float dx = rx - pb.x, dy = ry - pb.y, dz = rz - pb.z;
-                    const float r2 = __builtin_fmaf(dz, dz, __builtin_fmaf(dx, dx, dy * dy));
-                    if (c + u < len && r2 < 1.0f) {
-                        ql[ring(fill) * FSI_THREADS] = (unsigned)(b0 + c + u);
-                        fill++;
-                    }
+            for (int c = 0; c < 2; c++) {
+                unsigned b = mk.w[c];
+                while (wave_any(b != 0u)) {
+                    const int k = __builtin_clz(b | 1u);
+                    if (b && at >= 0 && at < FI_CAP)
+                        S.item[0][at] = (unsigned)h << 27 | (unsigned)(j + skip + 32 * c + k);
+                    at += b ? 1 : 0;
+                    b &= ~(0x80000000u >> k);
                 }
             }
             __builtin_amdgcn_wave_barrier();
-            continue;
-        }
-        // four candidates per iteration: four loads in flight per lane
-        for (int c = 0; wave_any(c < len); c += 4) {
-            if (wave_any(fill + 4 > FQ_V))
-#pragma unroll 1
-                for (int k = 0; k < FSI_DRAIN_STEPS; k++) drain_step();
-            float4 pb[4];
+            const int Tw = min(T - c0, FI_CAP);
+            auto in_of = [&](int q) {
+                // a lane past the list takes the first instance and solvent particle
+                const unsigned e = q < Tw ? S.item[0][q] : 0u, b = e & 0x7FFFFFFu;
+                const float4 hp = S.hp[e >> 27], hv = S.hv[e >> 27];
+                const f3v pb = pos_at(spos, b * 16u, 0), vb = pos_at(svel, b * 16u, 0);
+                const unsigned lid = (unsigned)__float_as_int(hp.w);
+                FsiIn o;
+                o.dx = hp.x - pb.x;
+                o.dy = hp.y - pb.y;
+                o.dz = hp.z - pb.z;
+                o.r2 = __builtin_fmaf(o.dz, o.dz, __builtin_fmaf(o.dx, o.dx, o.dy * o.dy));
+                o.dvx = hv.x - vb.x;
+                o.dvy = hv.y - vb.y;
+                o.dvz = hv.z - vb.z;
+                // mean0var1uu(seed, lid, b) before the logistic map (src/math/rnd/dev.h:65-72)
+                o.x = hv.w - low_discrepancy((float)(lid & 0x3FFu), (float)lid, (float)(b & 0x3FFu), (float)b);
+                return o;
+            };
+            auto put = [&](int q, const FsiIn &a, float x) {
+                const float3 f =
+                    dpd_pair<WR, EXACT>(K.par, a.dx, a.dy, a.dz, a.r2, a.dvx, a.dvy, a.dvz, x * R_SQRT2);
+                if (q < Tw) {
+                    S.item[0][q] = __float_as_uint(f.x);
+                    S.item[1][q] = __float_as_uint(f.y);
+                    S.item[2][q] = __float_as_uint(f.z);
+                }
+            };
+            for (int b = 0; b < Tw; b += 128) {
+                const FsiIn a0 = in_of(b + lane), a1 = in_of(b + 64 + lane);
+                float x0 = a0.x, x1 = a1.x;
+                logistic18x2(&x0, &x1);
+                put(b + lane, a0, x0);
+                put(b + 64 + lane, a1, x1);
+            }
+            __builtin_amdgcn_wave_barrier();
+            if (comp < 3) {
+                const unsigned *const it = S.item[comp];
+                const int ea = max(g0 - c0, 0), ee = min(g1 - c0, FI_CAP);
+                for (int k = ea; wave_any(k < ee); k += 8) {
+                    unsigned f[8];
 #pragma unroll
-            for (int u = 0; u < 4; u++) pb[u] = c + u < len ? K.spos[b0 + c + u] : make_float4(1e30f, 1e30f, 1e30f, 0.f);
+                    for (int u = 0; u < 8; u++) f[u] = it[k + u < ee ? k + u : 0];
 #pragma unroll
-            for (int u = 0; u < 4; u++) {
-                const float dx = rx - pb[u].x, dy = ry - pb[u].y, dz = rz - pb[u].z;
-                const float r2 = __builtin_fmaf(dz, dz, __builtin_fmaf(dx, dx, dy * dy));
-                if (c + u < len && r2 < 1.0f) {
-                    ql[ring(fill) * FSI_THREADS] = (unsigned)(b0 + c + u);
-                    fill++;
+                    for (int u = 0; u < 8; u++)
+                        if (k + u < ee) acc += __uint_as_float(f[u]);
                 }
             }
         }
+        if (sel < 0) break;
+        if (wave_any(nc > 64)) {
+            skip += 64;
+        } else {
+            skip = 0;
+            if (++sel == 9) break;
+        }
     }
-    while (wave_any(fill > 0)) drain_step();
-    if (active) {
-        float *o = sinst + 3 * (long)order[t];
-        o[0] = sx;
-        o[1] = sy;
-        o[2] = sz;
-    }
+    const int g = lane % FI_HOMES, comp = lane / FI_HOMES;
+    if (comp < 3 && first + g < n) sinst[3 * (long)order[first + g] + comp] = acc;
     if (pairs) {
-        unsigned long long c = (unsigned long long)np;
-        for (int d = 32; d >= 1; d >>= 1) c += __shfl_xor(c, d, 64);
-        if ((threadIdx.x & 63) == 0 && c) atomicAdd(pairs, c);
+        if (lane == 0) count[w] = np;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            int c = 0;
+            for (int k = 0; k < FI_WAVES; k++) c += count[k];
+            if (c) atomicAdd(pairs, (unsigned long long)c);
+        }
     }
 }
 
@@ -460,7 +460,7 @@ void fsi_free(FsiBufs *f) {
 }
 
 int fsi_forces(hipStream_t s, FsiBufs *f, int ns, const float4 *spos, const float4 *svel, const int *starts,
-               int no, const float *opp, const udx_pair_dpd &p, const float *seeds_dev, float *fo, float *fs,
+               const int *bstarts, int sub, int no, const float *opp, const udx_pair_dpd &p, const float *seeds_dev, float *fo, float *fs,
                int fs_stride, unsigned long long *pairs, int exact) {
     const Box &b = f->box;
     UDX_CHECK(no >= 0 && no <= f->max_obj, UDX_ECAP, "fsi: %d membrane vertices above the capacity %d", no,
@@ -488,12 +488,14 @@ int fsi_forces(hipStream_t s, FsiBufs *f, int ns, const float4 *spos, const floa
     K.spos = spos;
     K.svel = svel;
     K.starts = starts;
+    K.bstarts = bstarts;
+    K.sub = sub;
     K.par = DpdPar{p.a, p.g, p.s, p.spow};
     K.seeds = seeds_dev;
 #define UDX_FSI_LAUNCH(WR, EX)                                                                                  \
     do {                                                                                                        \
-        hipLaunchKernelGGL((k_fsi_instance<WR, EX>), dim3(ceil_div(nmax, FSI_THREADS)), dim3(FSI_THREADS), 0,  \
-                           s, K, f->cl.starts + nc, f->inst_sorted, f->meta_sorted, f->cl.order, f->sinst,      \
+        hipLaunchKernelGGL((k_fsi_instance<WR, EX>), dim3(ceil_div(nmax, FI_HOMES * FI_WAVES)),                 \
+                           dim3(64 * FI_WAVES), 0, s, K, f->cl.starts + nc, f->inst_sorted, f->meta_sorted, f->cl.order, f->sinst,      \
                            pairs);                                                                              \
         if (ns > 0)                                                                                             \
             hipLaunchKernelGGL((k_fsi_solvent<WR, EX>), dim3(ceil_div(ns, FSI_THREADS)), dim3(FSI_THREADS), 0,  \
@@ -587,7 +589,7 @@ int udx_fsi_bind_solvent(udx_fsi *q, const float *pp, float *ff, int n, const in
     if (n > q->cap_s) {
         dev_free(q->spos);
         dev_free(q->svel);
-        UDX_TRY(dev_alloc(&q->spos, (size_t)n));
+        UDX_TRY(dev_alloc(&q->spos, (size_t)n + POS_PAD));
         UDX_TRY(dev_alloc(&q->svel, (size_t)n));
         q->cap_s = n;
     }
@@ -606,7 +608,7 @@ int udx_fsi_apply_seeds(udx_fsi *q, const udx_pair_dpd *p, int no, const float *
     if (no == 0) return UDX_OK;
     UDX_HIP(hipMemcpyAsync(q->seeds_dev, seeds, 2 * sizeof(float), hipMemcpyHostToDevice, s));
     if (q->ns > 0) UDX_TRY(aos_to_f4(s, q->ns, q->spp, q->spos, q->svel));
-    UDX_TRY(fsi_forces(s, &q->f, q->ns, q->spos, q->svel, q->starts, no, opp, *p, q->seeds_dev, off, q->sff, 3,
+    UDX_TRY(fsi_forces(s, &q->f, q->ns, q->spos, q->svel, q->starts, nullptr, 1, no, opp, *p, q->seeds_dev, off, q->sff, 3,
                        q->pairs_dev, q->mode == UDX_MODE_EXACT));
     // the seeds live on the host stack: wait for the copy before returning
     UDX_HIP(hipStreamSynchronize(s));

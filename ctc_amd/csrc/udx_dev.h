@@ -263,6 +263,135 @@ __device__ __forceinline__ int frag_cell(int dx, int dy, int dz, int cx, int cy,
 // ---------------------------------------------------------------- waves
 __device__ __forceinline__ bool wave_any(bool p) { return __any(p); }
 
+// v summed over the lanes up to this one
+__device__ __forceinline__ int wave_scan_add(int v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);   // row_shr:1
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);   // row_bcast:15
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);   // row_bcast:31
+    return v;
+}
+
+// smallest and largest value over the wave's lanes
+__device__ __forceinline__ int wave_min(int v) {
+    v = min(v, __builtin_amdgcn_update_dpp(0x7fffffff, v, 0x111, 0xf, 0xf, false));
+    v = min(v, __builtin_amdgcn_update_dpp(0x7fffffff, v, 0x112, 0xf, 0xf, false));
+    v = min(v, __builtin_amdgcn_update_dpp(0x7fffffff, v, 0x114, 0xf, 0xf, false));
+    v = min(v, __builtin_amdgcn_update_dpp(0x7fffffff, v, 0x118, 0xf, 0xf, false));
+    v = min(v, __builtin_amdgcn_update_dpp(0x7fffffff, v, 0x142, 0xa, 0xf, false));
+    v = min(v, __builtin_amdgcn_update_dpp(0x7fffffff, v, 0x143, 0xc, 0xf, false));
+    return __builtin_amdgcn_readlane(v, 63);
+}
+__device__ __forceinline__ int wave_max(int v) { return -wave_min(-v); }
+
+// ---------------------------------------------------------------- candidates
+// Arrays typed as global memory: pointers read from a table in memory are
+// otherwise generic, and generic (flat) loads count against the LDS wait
+// counter as well.
+#define UDX_GLOBAL __attribute__((address_space(1)))
+typedef float f4v __attribute__((ext_vector_type(4)));
+typedef float f3v __attribute__((ext_vector_type(3)));   // 16 B in memory; loads read 12
+
+template <class T>
+__device__ __forceinline__ UDX_GLOBAL T *gptr(T *p) {
+    return (UDX_GLOBAL T *)p;
+}
+
+// x, y, z of the entry at a byte offset, plus K entries folded into the load.
+// The 32-bit offset (indices stay below 2^27) goes into the load beside the
+// base; a signed index takes five more instructions per particle to widen.
+__device__ __forceinline__ f3v pos_at(const UDX_GLOBAL f4v *p, unsigned byte, int k) {
+    return *(const UDX_GLOBAL f3v *)((const UDX_GLOBAL char *)p + (size_t)byte + 16 * k);
+}
+
+// Candidate window along x.  With x-slab starts a row run [x0, x1] of cells
+// (wrap wx) is cut to the slabs that can hold a particle within the cutoff:
+// a candidate at y-z distance >= d from the particle has |dx| < sqrt(1 - d^2).
+// The bound is conservative for the float pair test: the y-z gaps g are
+// lowered and the half-width raised by WIN_MARGIN (above the rounding of
+// the particle's periodic shift for boxes up to 2048 cells) and 1 + 1e-5
+// stands for the cutoff, so every candidate the test would accept lies in
+// the window.  hw < 0: no particle of the row is within the cutoff.
+constexpr float WIN_MARGIN = 1.0f / 4096.0f;
+
+__device__ __forceinline__ float row_halfwidth(int dy, int dz, float fy, float fz) {
+    float gy = dy == 0 ? 0.f : (dy < 0 ? fy : 1.f - fy);
+    float gz = dz == 0 ? 0.f : (dz < 0 ? fz : 1.f - fz);
+    gy = fmaxf(gy - WIN_MARGIN, 0.f);
+    gz = fmaxf(gz - WIN_MARGIN, 0.f);
+    const float w2 = 1.00001f - gy * gy - gz * gz;
+    return w2 < 0.f ? -1.f : __builtin_amdgcn_sqrtf(w2) + WIN_MARGIN;
+}
+
+// candidates of the run [x0, x1] of the row starting at cell `base`, for a
+// particle in column c of the run's frame (its own column less the wrap times
+// the box side), fx into its cell: index range [*j, *j + *n).  The window is
+// counted in slabs from the particle's cell, so floats hold it exactly enough
+// for the margin (slabs counted from the box edge need doubles, three times
+// the issue cycles).
+__device__ __forceinline__ void run_range(const UDX_GLOBAL int *starts, const UDX_GLOBAL int *bstarts, int sub,
+                                          int base, int x0, int x1, int c, float fx, float hw, int *j, int *n) {
+    const UDX_GLOBAL int *st = starts;
+    int lo = base + x0, hi = base + x1;
+    if (bstarts) {
+        const int S = sub;
+        st = bstarts;
+        lo = max(c * S + (int)__builtin_floorf((fx - hw) * (float)S), x0 * S);
+        hi = min(c * S + (int)__builtin_floorf((fx + hw) * (float)S), x1 * S + S - 1);
+        if (!(hw >= 0.f) || lo > hi) {
+            *j = 0;
+            *n = 0;
+            return;
+        }
+        lo += base * S;
+        hi += base * S;
+    }
+    *j = st[lo];
+    *n = st[hi + 1] - *j;
+}
+
+// hits of up to 64 candidates as bits, candidate k at bit 31 - (k mod 32) of
+// word k / 32: the sign of r2 - 1, shifted in from the right.  at(k) reads the
+// lane's candidate k, for k up to seven past the last one.
+struct Mask64 {
+    unsigned w[2];
+};
+template <class At>
+__device__ __forceinline__ Mask64 test64(int n, float ax, float ay, float az, At at) {
+    Mask64 m{{0u, 0u}};
+#pragma unroll
+    for (int c = 0; c < 2; c++) {
+        if (!wave_any(n > 32 * c)) break;
+        unsigned b = 0;
+        int sh = 32;
+        f3v q[4], nx[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) q[u] = at(32 * c + u);
+#pragma unroll
+        for (int g = 0; g < 8; g++) {
+            if (g && !wave_any(n > 32 * c + 4 * g)) break;
+            if (g < 7)
+#pragma unroll
+                for (int u = 0; u < 4; u++) nx[u] = at(32 * c + 4 * (g + 1) + u);
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                const float dx = ax - q[u].x, dy = ay - q[u].y, dz = az - q[u].z;
+                const float r2 = __builtin_fmaf(dz, dz, __builtin_fmaf(dx, dx, dy * dy));
+                b = __builtin_amdgcn_alignbit(b, __float_as_uint(r2 - 1.0f), 31);
+            }
+            sh -= 4;
+#pragma unroll
+            for (int u = 0; u < 4; u++) q[u] = nx[u];
+        }
+        b <<= sh & 31;
+        const int left = n - 32 * c;
+        m.w[c] = left >= 32 ? b : (left > 0 ? b & ~(0xFFFFFFFFu >> left) : 0u);
+    }
+    return m;
+}
+
 // ---------------------------------------------------------------- SDF
 // wall margin in cells (XWM/YWM/ZWM, src/inc/def.h:15-18)
 constexpr int WALL_MARGIN = 6;

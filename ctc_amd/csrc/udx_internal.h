@@ -319,9 +319,10 @@ struct FsiBufs {
 int fsi_alloc(FsiBufs *f, const Box &b, int max_obj);
 void fsi_free(FsiBufs *f);
 // +f on the vertices (fo, stride 3) and -f on the solvent (fs, fs_stride),
-// both ADDED; seeds_dev = [bulk, halo]
+// both ADDED; spos has POS_PAD entries past its particles; bstarts: x-slab
+// starts of the solvent list (sub per cell) or null; seeds_dev = [bulk, halo]
 int fsi_forces(hipStream_t s, FsiBufs *f, int ns, const float4 *spos, const float4 *svel, const int *starts,
-               int no, const float *opp, const udx_pair_dpd &p, const float *seeds_dev, float *fo, float *fs,
+               const int *bstarts, int sub, int no, const float *opp, const udx_pair_dpd &p, const float *seeds_dev, float *fo, float *fs,
                int fs_stride, unsigned long long *pairs, int exact);
 FsiBufs *fsi_bufs(udx_fsi *q);
 udx_ctx *fsi_ctx(const udx_fsi *q);

@@ -9,6 +9,7 @@ import numpy as np
 import pytest
 
 import oracle as O
+from oracle import rbc as R
 from oracle import wall as W
 
 pytestmark = pytest.mark.gpu
@@ -143,3 +144,30 @@ def test_walls_bit_exact(ctx, rho):
     assert np.array_equal(got.view(np.uint32), cur.view(np.uint32))
     w.close()
     q.close()
+
+
+@pytest.mark.parametrize("rho,nv", [(60, 40), (60, 1), (12, 300), (2, 15)])
+def test_vertex_side_bit_exact(ctx, rho, nv):
+    """solvent-vertex pairs at densities where a vertex's rows hold 180
+    candidates and a wave's pairs fill its list several times over, last waves
+    with one vertex, vertices outside the box on every side"""
+    L = (6, 4, 8)
+    say("vertex side", rho, nv)
+    starts, _, srt, _ = O.clist_build(L, particles(L, rho * 6 * 4 * 8, 8))
+    rng = np.random.default_rng(9)
+    opp = np.zeros((nv, 6), np.float32)
+    opp[:, :3] = rng.uniform(-0.65, 0.65, (nv, 3)) * np.array(L)
+    opp[:, 3:] = rng.normal(0, 0.1, (nv, 3))
+    par = (2.6666667, 8.0, O.dpd_sigma(0.0444, 8.0, 5e-4), 0.25)
+    seeds = np.array([0.31, 0.77], np.float32)
+    fo0, fs0 = np.ones((nv, 3), np.float32), np.zeros((len(srt), 3), np.float32)
+    fo, fs, n = R.fsi_forces(L, srt, starts, opp, par, seeds, fo0, fs0)
+    f = U.Fsi(ctx, L, nv, exact=True)
+    sd, fd, st = torch.as_tensor(srt).cuda(), torch.as_tensor(fs0).cuda(), torch.as_tensor(starts).cuda()
+    f.bind_solvent(sd, fd, U._ptr(st))
+    od = torch.as_tensor(fo0).cuda()
+    f.apply(U.PairDpd(*par), torch.as_tensor(opp).cuda(), od, seeds=seeds)
+    assert f.pairs() == n and n > 0
+    assert np.array_equal(host(od).view(np.uint32), fo.view(np.uint32))
+    assert np.array_equal(host(fd).view(np.uint32), fs.view(np.uint32))
+    f.close()
