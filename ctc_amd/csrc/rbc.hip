@@ -154,6 +154,82 @@ __global__ __launch_bounds__(RBC_THREADS) void k_rbc_force(RbcK K, const float *
     o[2] += (float)f.z;
 }
 
+// A lane per ring slot: a wave takes as many vertices as their slots fit its
+// lanes (ten of degree 6), each lane evaluates its slot's triangle, viscous and
+// two dihedral terms, and lanes of the vertex add the slots' terms in slot
+// order from LDS, one sum each (membrane and bending, x y z), in double; their
+// total is added to the float force once.  The order of the additions is that
+// of a walk over the ring, which k_rbc_force makes slot after slot (one cell of
+// 642 vertices: 21 -> 7.3 us); the exchange through LDS costs more than it
+// hides where k_rbc_force fills the chip by itself (164 thousand vertices: 47 ->
+// 60 us), rbc_force_small() has the line.
+constexpr int RF_WAVES = 4;
+__global__ __launch_bounds__(64 * RF_WAVES) void k_rbc_force_slots(RbcK K, const float *pp, const double *av, float *ff) {
+    __shared__ double term[RF_WAVES][12][64];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    double(*const tm)[64] = term[w];
+    const int G = K.md < 64 ? K.md : 64, per = 64 / G;   // lanes per vertex, vertices per wave
+    const int lv = lane / G, js = lane % G;
+    const int v = (blockIdx.x * RF_WAVES + w) * per + lv;
+    const bool active = lv < per && v < K.nc * K.nv;
+    const int cell = active ? v / K.nv : 0, off = cell * K.nv, vt = active ? v - off : 0;
+    const double A = av[2 * cell], V = av[2 * cell + 1];
+    const D3 r0 = rpos(pp, off + vt), u0 = rvel(pp, off + vt);
+    // this lane's sums: js and, for vertices of fewer than six slots, js + G, js + 2 G, ...
+    double acc[6] = {0, 0, 0, 0, 0, 0};
+    for (int j0 = 0; j0 < K.md; j0 += G) {
+        const int j = j0 + js;
+        D3 t[4] = {mk(0, 0, 0), mk(0, 0, 0), mk(0, 0, 0), mk(0, 0, 0)};
+        int i1, i2, i3, i4;
+        if (active && j < K.md && adj_map(K, vt, j, &i1, &i2, &i3, &i4)) {
+            const int s = vt * K.md + j;
+            const double l0 = K.ll ? (double)K.ll[s] : (double)K.l0;
+            const double a0 = K.aa ? (double)K.aa[s] : (double)K.a0;
+            const D3 r1 = rpos(pp, i1 + off), r2 = rpos(pp, i2 + off);
+            t[0] = ftri(K, r0, r1, r2, l0, a0, A, V);
+            t[1] = fvisc(K, r0, r1, u0, rvel(pp, i1 + off));
+            if (K.bending) {
+                const D3 r3 = rpos(pp, i3 + off), r4 = rpos(pp, i4 + off);
+                t[2] = dih<1>(K, r0, r2, r1, r4);
+                t[3] = dih<2>(K, r1, r0, r2, r3);
+            }
+        }
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            tm[3 * k][lane] = t[k].x;
+            tm[3 * k + 1][lane] = t[k].y;
+            tm[3 * k + 2][lane] = t[k].z;
+        }
+        __builtin_amdgcn_wave_barrier();
+        // sum c: component c % 3 of the membrane terms (c < 3) or the bending
+        // terms; a slot without a triangle left zeros, which change nothing
+        if (lv < per)
+#pragma unroll
+            for (int q = 0; q < 6; q++) {
+                const int c = js + q * G;
+                if (c >= 6) break;
+                const double *const x = tm[c % 3 + 6 * (c / 3)], *const y = tm[c % 3 + 6 * (c / 3) + 3];
+                for (int s = 0; s < G; s++) {
+                    acc[q] += x[lv * G + s];
+                    acc[q] += y[lv * G + s];
+                }
+            }
+    }
+    __builtin_amdgcn_wave_barrier();
+    if (lv < per)
+#pragma unroll
+        for (int q = 0; q < 6; q++)
+            if (js + q * G < 6) tm[js + q * G][lv] = acc[q];
+    __builtin_amdgcn_wave_barrier();
+    for (int c = js; c < 3 && active; c += G) ff[3 * (long)v + c] += (float)(tm[c][lv] + tm[c + 3][lv]);
+}
+
+// A lane per slot up to 65536 vertices, one wave per SIMD of k_rbc_force: force,
+// loads and move of n cells of 642 vertices, lane per vertex -> per slot, 16:
+// 33.5 -> 23.9 us, 64: 44.2 -> 34.5, 96: 45.3 -> 41.6, 128: 47.8 -> 49.6.
+bool rbc_force_small(int n) { return n <= 65536; }
+
 // per cell [area, volume] in FP64: one block per cell, fixed-order tree
 // reduction (src/rbc/force/area_volume/dev/main.h:1-46)
 constexpr int AV_THREADS = 256;
@@ -786,8 +862,14 @@ int udx_rbc_force_apply(udx_rbc *r, const udx_rbc_params *p, float dt, int nc, c
     K.cphi = std::cos(phi);
     K.bending = r->bending;
     const int n = nc * r->nv;
-    hipLaunchKernelGGL(k_rbc_force, dim3(ceil_div(n, RBC_THREADS)), dim3(RBC_THREADS), 0, r->ctx->stream, K, pp,
-                       r->av, ff);
+    if (rbc_force_small(n)) {
+        const int per = 64 / (r->md < 64 ? r->md : 64);   // vertices per wave
+        hipLaunchKernelGGL(k_rbc_force_slots, dim3(ceil_div(n, per * RF_WAVES)), dim3(64 * RF_WAVES), 0,
+                           r->ctx->stream, K, pp, r->av, ff);
+    } else {
+        hipLaunchKernelGGL(k_rbc_force, dim3(ceil_div(n, RBC_THREADS)), dim3(RBC_THREADS), 0, r->ctx->stream, K, pp,
+                           r->av, ff);
+    }
     UDX_LAUNCHED();
     // bending_apply (src/rbc/force/imp/forces.h:54) for the Juelicher model
     if (r->juelicher) UDX_TRY(jul_apply(r->ctx->stream, r->jt, nc, pp, ff));
