@@ -17,6 +17,7 @@ namespace udx {
 namespace {
 
 constexpr int CNT_THREADS = 128;
+constexpr int CNT_FORCE = 64;   // k_cnt_force: a wave per block, so that few vertices reach more CUs
 
 struct DpdLj {
     float a, g, s, spow, ljs, lje;
@@ -165,8 +166,57 @@ struct CntK {
     const int *starts, *order, *hstarts, *horder, *flags, *pos;
 };
 
-__global__ __launch_bounds__(CNT_THREADS) void k_cnt_force(CntK K, float *ff, unsigned long long *pairs) {
-    const int v = blockIdx.x * CNT_THREADS + threadIdx.x;
+// the 9 rows of the block of cells around c (z, then y, ascending), each a
+// contiguous run of the cell list: its at most 3 cells follow one another, so
+// a row takes two loads of starts where the cells took six; every row's bounds
+// are loaded before the first is used
+struct Rows {
+    int s[9], e[9];
+};
+__device__ __forceinline__ Rows block_rows(const int *starts, const int L[3], const int c[3]) {
+    Rows w;
+    const int x0 = max(c[0] - 1, 0), x1 = min(c[0] + 1, L[0] - 1);
+#pragma unroll
+    for (int k = 0; k < 9; k++) {
+        const int z = c[2] - 1 + k / 3, y = c[1] - 1 + k % 3;
+        w.s[k] = w.e[k] = 0;
+        if (x0 > x1 || y < 0 || y >= L[1] || z < 0 || z >= L[2]) continue;
+        const int row = L[0] * (y + L[1] * z);
+        w.s[k] = starts[row + x0];
+        w.e[k] = starts[row + x1 + 1];
+    }
+    return w;
+}
+
+// the points of a block's rows in order, four loads in flight; f(index, point)
+// for those closer than 1 to a (or not comparable: cnt_pair's own test)
+template <class F>
+__device__ __forceinline__ void near_points(const Rows &w, const int *order, const float *pp, const float *a, F f) {
+#pragma unroll
+    for (int k = 0; k < 9; k++)
+        for (int s = w.s[k]; s < w.e[k]; s += 4) {
+            int u[4];
+            float r[4][6];
+#pragma unroll
+            for (int t = 0; t < 4; t++) u[t] = order[min(s + t, w.e[k] - 1)];
+#pragma unroll
+            for (int t = 0; t < 4; t++) load6(pp, u[t], r[t]);
+#pragma unroll
+            for (int t = 0; t < 4; t++) {
+                const float dx = a[0] - r[t][0], dy = a[1] - r[t][1], dz = a[2] - r[t][2];
+                const float r2 = __builtin_fmaf(dz, dz, __builtin_fmaf(dx, dx, dy * dy));
+                if (s + t < w.e[k] && !(r2 >= 1.0f)) f(u[t], r[t]);
+            }
+        }
+}
+
+// Bound by the latency of its loads (a few thousand vertices leave most CUs
+// without a wave): one chain starts -> order -> vertex per four candidates of
+// a row, the noise drawn for close pairs only, and the 26 flags read only by
+// the vertices outside the domain, the only ones with images.  8 red cells of
+// 498 vertices: 41 us, against 87 with a load chain per cell and candidate.
+__global__ __launch_bounds__(CNT_FORCE) void k_cnt_force(CntK K, float *ff, unsigned long long *pairs) {
+    const int v = blockIdx.x * CNT_FORCE + threadIdx.x;
     if (v >= K.n) return;
     const int L[3] = {K.Lx, K.Ly, K.Lz};
     float rv[6];
@@ -176,69 +226,47 @@ __global__ __launch_bounds__(CNT_THREADS) void k_cnt_force(CntK K, float *ff, un
     float acc[3] = {0, 0, 0};
     unsigned np = 0;
     // bulk pairs
-    for (int z = cv[2] - 1; z <= cv[2] + 1; z++)
-        for (int y = cv[1] - 1; y <= cv[1] + 1; y++)
-            for (int x = cv[0] - 1; x <= cv[0] + 1; x++) {
-                if (x < 0 || x >= L[0] || y < 0 || y >= L[1] || z < 0 || z >= L[2]) continue;
-                const int cid = x + L[0] * (y + L[1] * z);
-                for (int s = K.starts[cid]; s < K.starts[cid + 1]; s++) {
-                    const int u = K.order[s];
-                    if (u == v) continue;
-                    float ru[6], f[3];
-                    load6(K.pp, u, ru);
-                    const int hi = u > v ? u : v, lo = u > v ? v : u;
-                    const float rnd = mean0var1ii(K.seed_bulk, hi, lo);
-                    if (!(v == hi ? cnt_pair(K.p, rv, ru, rnd, f) : cnt_pair(K.p, ru, rv, rnd, f))) continue;
-                    if (v == hi) {
-                        acc[0] += f[0]; acc[1] += f[1]; acc[2] += f[2];
-                        np++;
-                    } else {
-                        acc[0] -= f[0]; acc[1] -= f[1]; acc[2] -= f[2];
-                    }
-                }
-            }
+    const Rows wb = block_rows(K.starts, L, cv), wh = block_rows(K.hstarts, L, cv);
+    near_points(wb, K.order, K.pp, rv, [&](int u, const float *ru) {
+        if (u == v) return;
+        float f[3];
+        const int hi = u > v ? u : v, lo = u > v ? v : u;
+        const float rnd = mean0var1ii(K.seed_bulk, hi, lo);
+        if (!(v == hi ? cnt_pair(K.p, rv, ru, rnd, f) : cnt_pair(K.p, ru, rv, rnd, f))) return;
+        if (v == hi) {
+            acc[0] += f[0]; acc[1] += f[1]; acc[2] += f[2];
+            np++;
+        } else {
+            acc[0] -= f[0]; acc[1] -= f[1]; acc[2] -= f[2];
+        }
+    });
     // images acting on v
-    for (int z = cv[2] - 1; z <= cv[2] + 1; z++)
-        for (int y = cv[1] - 1; y <= cv[1] + 1; y++)
-            for (int x = cv[0] - 1; x <= cv[0] + 1; x++) {
-                if (x < 0 || x >= L[0] || y < 0 || y >= L[1] || z < 0 || z >= L[2]) continue;
-                const int cid = x + L[0] * (y + L[1] * z);
-                for (int s = K.hstarts[cid]; s < K.hstarts[cid + 1]; s++) {
-                    const int h = K.horder[s];
-                    float ri[6], f[3];
-                    load6(K.img, h, ri);
-                    bool ok = true;
-                    for (int c = 0; c < 3; c++) {
-                        const int ch = ccell(ri[c], L[c], false);
-                        if (cv[c] < ch - 1 || cv[c] > ch + 1) ok = false;
-                    }
-                    if (!ok) continue;
-                    if (!cnt_pair(K.p, ri, rv, mean0var1ii(K.seed_halo, h, v), f)) continue;
-                    acc[0] -= f[0]; acc[1] -= f[1]; acc[2] -= f[2];
-                }
-            }
-    // v's own images against the vertices of their blocks
-    for (int i = 0; i < 26; i++) {
+    near_points(wh, K.horder, K.img, rv, [&](int h, const float *ri) {
+        float f[3];
+        for (int c = 0; c < 3; c++) {
+            const int ch = ccell(ri[c], L[c], false);
+            if (cv[c] < ch - 1 || cv[c] > ch + 1) return;
+        }
+        if (!cnt_pair(K.p, ri, rv, mean0var1ii(K.seed_halo, h, v), f)) return;
+        acc[0] -= f[0]; acc[1] -= f[1]; acc[2] -= f[2];
+    });
+    // v's own images against the vertices of their blocks; sends() gives no
+    // vertex inside the domain an image
+    bool out = false;
+    for (int c = 0; c < 3; c++) out |= !(rv[c] >= (float)(-L[c] / 2)) || rv[c] >= (float)(L[c] / 2);
+    for (int i = 0; out && i < 26; i++) {
         if (!K.flags[i * K.n + v]) continue;
         const int h = K.pos[i * K.n + v];
         float ri[6];
         load6(K.img, h, ri);
         int ch[3];
         for (int c = 0; c < 3; c++) ch[c] = ccell(ri[c], L[c], false);
-        for (int z = ch[2] - 1; z <= ch[2] + 1; z++)
-            for (int y = ch[1] - 1; y <= ch[1] + 1; y++)
-                for (int x = ch[0] - 1; x <= ch[0] + 1; x++) {
-                    if (x < 0 || x >= L[0] || y < 0 || y >= L[1] || z < 0 || z >= L[2]) continue;
-                    const int cid = x + L[0] * (y + L[1] * z);
-                    for (int s = K.starts[cid]; s < K.starts[cid + 1]; s++) {
-                        const int b = K.order[s];
-                        float rb[6], f[3];
-                        load6(K.pp, b, rb);
-                        if (!cnt_pair(K.p, ri, rb, mean0var1ii(K.seed_halo, h, b), f)) continue;
-                        acc[0] += f[0]; acc[1] += f[1]; acc[2] += f[2];
-                        np++;
-                    }
-                }
+        near_points(block_rows(K.starts, L, ch), K.order, K.pp, ri, [&](int b, const float *rb) {
+            float f[3];
+            if (!cnt_pair(K.p, ri, rb, mean0var1ii(K.seed_halo, h, b), f)) return;
+            acc[0] += f[0]; acc[1] += f[1]; acc[2] += f[2];
+            np++;
+        });
     }
     float *o = ff + 3 * (size_t)v;
     o[0] += acc[0];
@@ -318,7 +346,7 @@ int cnt_forces(hipStream_t s, udx_cnt *c, const udx_pair_dpd_lj &pr, int n, cons
                        c->hstarts, c->hcounts, c->hfill, c->horder);
     CntK K{n, L[0], L[1], L[2], {pr.a, pr.g, pr.s, pr.spow, pr.ljs, pr.lje}, seed_bulk, seed_halo, pp, c->img,
            c->starts, c->order, c->hstarts, c->horder, c->flags, c->pos};
-    hipLaunchKernelGGL(k_cnt_force, dim3(ceil_div(n, CNT_THREADS)), dim3(CNT_THREADS), 0, s, K, ff, c->pairs);
+    hipLaunchKernelGGL(k_cnt_force, dim3(ceil_div(n, CNT_FORCE)), dim3(CNT_FORCE), 0, s, K, ff, c->pairs);
     UDX_LAUNCHED();
     return UDX_OK;
 }

@@ -171,3 +171,29 @@ def test_vertex_side_bit_exact(ctx, rho, nv):
     assert np.array_equal(host(od).view(np.uint32), fo.view(np.uint32))
     assert np.array_equal(host(fd).view(np.uint32), fs.view(np.uint32))
     f.close()
+
+
+@pytest.mark.parametrize("L,n", [((2, 3, 4), 257), ((6, 4, 8), 64), ((6, 4, 8), 1500), ((1, 5, 2), 65), ((16, 16, 16), 1)])
+def test_contact_bit_exact(ctx, L, n):
+    """membrane contact: rows of cells with none, one and many points (four are
+    loaded at a time), boxes thinner than a block of cells, vertices on the
+    faces and outside the box on every side, last waves with one vertex"""
+    say("contact", L, n)
+    rng = np.random.default_rng(n)
+    pp = np.zeros((n, 6), np.float32)
+    pp[:, :3] = rng.uniform(-0.7, 0.7, (n, 3)) * np.array(L)
+    for c in range(3):
+        pp[c::11, c] = L[c] // 2
+        pp[c + 3::11, c] = -(L[c] // 2)
+    pp[:, 3:] = rng.normal(0, 0.3, (n, 3))
+    if n > 9:
+        pp[n - 1, :3] = pp[0, :3]
+    par, sb, sh = (20.0, 8.0, 3.0, 0.25, 0.3, 1.0), np.float32(0.123), np.float32(0.456)
+    ff = rng.normal(0, 1, (n, 3)).astype(np.float32)
+    want, npair = R.cnt_forces(L, pp, par, sb, sh, ff=ff.copy())
+    c = U.Cnt(ctx, L, n)
+    fd = torch.as_tensor(ff).cuda()
+    c.apply(U.PairDpdLj(*par), torch.as_tensor(pp).cuda(), fd, seeds=(sb, sh))
+    assert c.pairs() == npair and (npair > 0 or n == 1)
+    assert np.array_equal(host(fd).view(np.uint32), want.view(np.uint32))
+    c.close()
