@@ -213,8 +213,8 @@ __device__ __forceinline__ void near_points(const Rows &w, const int *order, con
 // Bound by the latency of its loads (a few thousand vertices leave most CUs
 // without a wave): one chain starts -> order -> vertex per four candidates of
 // a row, the noise drawn for close pairs only, and the 26 flags read only by
-// the vertices outside the domain, the only ones with images.  8 red cells of
-// 498 vertices: 41 us, against 87 with a load chain per cell and candidate.
+// the vertices outside the domain, the only ones with images.  32 red cells
+// of 162 vertices: 41 us, against 87 with a load chain per cell and candidate.
 __global__ __launch_bounds__(CNT_FORCE) void k_cnt_force(CntK K, float *ff, unsigned long long *pairs) {
     const int v = blockIdx.x * CNT_FORCE + threadIdx.x;
     if (v >= K.n) return;

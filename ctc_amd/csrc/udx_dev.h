@@ -353,8 +353,10 @@ __device__ __forceinline__ void run_range(const UDX_GLOBAL int *starts, const UD
 }
 
 // hits of up to 64 candidates as bits, candidate k at bit 31 - (k mod 32) of
-// word k / 32: the sign of r2 - 1, shifted in from the right.  at(k) reads the
-// lane's candidate k, for k up to seven past the last one.
+// word k / 32: the sign of |r2| - 1, shifted in from the right (the modulus, an
+// input modifier without a cost, clears the sign that a NaN can carry: a
+// position that is not a number hits nothing, as with r2 < 1).  at(k) reads the
+// lane's candidate k, k below 64: at most 63 past the lane's first.
 struct Mask64 {
     unsigned w[2];
 };
@@ -379,7 +381,7 @@ __device__ __forceinline__ Mask64 test64(int n, float ax, float ay, float az, At
             for (int u = 0; u < 4; u++) {
                 const float dx = ax - q[u].x, dy = ay - q[u].y, dz = az - q[u].z;
                 const float r2 = __builtin_fmaf(dz, dz, __builtin_fmaf(dx, dx, dy * dy));
-                b = __builtin_amdgcn_alignbit(b, __float_as_uint(r2 - 1.0f), 31);
+                b = __builtin_amdgcn_alignbit(b, __float_as_uint(__builtin_fabsf(r2) - 1.0f), 31);
             }
             sh -= 4;
 #pragma unroll

@@ -197,3 +197,27 @@ def test_contact_bit_exact(ctx, L, n):
     assert c.pairs() == npair and (npair > 0 or n == 1)
     assert np.array_equal(host(fd).view(np.uint32), want.view(np.uint32))
     c.close()
+
+
+@pytest.mark.parametrize("nan", [0x7FC00000, 0xFFC00000])
+@pytest.mark.parametrize("c", [0, 1, 2])
+def test_not_a_number_hits_nothing(ctx, nan, c):
+    """a particle whose position is not a number, of either sign, acts on no
+    other one: their forces are those with the particle far away"""
+    L, rho, k = (8, 6, 8), 8, 1500
+    say("not a number", hex(nan), c)
+    starts, _, srt, _ = O.clist_build(L, particles(L, rho * 8 * 6 * 8, 4))
+    sd, out = torch.as_tensor(starts).cuda(), []
+    for bits in (np.float32(1e6).view(np.uint32), np.uint32(nan)):
+        pp = srt.copy()
+        pp.view(np.uint32)[k, c] = bits
+        f = U.FluForces(ctx, L, len(pp))
+        f.prepare(torch.as_tensor(pp).cuda())
+        ff = torch.zeros((len(pp), 3), device="cuda")
+        f.apply(U.PairDpd(25.0, 4.5, O.dpd_sigma(0.5, 4.5, 1e-3), 0.25), U._ptr(sd), ff,
+                seeds=O.seeds_table(1)[0])
+        out.append((np.delete(host(ff), k, 0), f.pairs()))
+        f.close()
+    assert np.isfinite(out[0][0]).all() and out[0][1] > 0
+    assert out[0][1] == out[1][1]
+    assert np.array_equal(out[0][0].view(np.uint32), out[1][0].view(np.uint32))
