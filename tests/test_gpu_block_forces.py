@@ -221,3 +221,34 @@ def test_not_a_number_hits_nothing(ctx, nan, c):
     assert np.isfinite(out[0][0]).all() and out[0][1] > 0
     assert out[0][1] == out[1][1]
     assert np.array_equal(out[0][0].view(np.uint32), out[1][0].view(np.uint32))
+
+
+@pytest.mark.parametrize("rho,order", [(3, "cells"), (30, "cells"), (30, "shuffled"), (45, "cells"), (45, "one")])
+def test_wall_rows_bit_exact(ctx, rho, order):
+    """wall forces by a launch of their own: rows that a wave stages and rows
+    too long for it (density 45: 135 candidates a run; particles out of cell
+    order), runs of more than 64, one particle"""
+    L = (7, 6, 16)
+    say("wall rows", rho, order)
+    ext, N = np.array(L, np.float32), (48, 48, 48)
+    D = W.plane_channel_sdf(L, 48, 4.0)
+    q, ref = U.Sdf(ctx, L, ext=ext, N=N, D=D), W.Sdf(L, ext, N, D.ravel())
+    pp = particles(L, rho * 7 * 6 * 16, 6)
+    d = torch.as_tensor(pp).cuda()
+    w = U.Wall(ctx, q, d)
+    _, frozen = ref.freeze(pp)
+    wst, _, wpp, _ = O.clist_build(W.margin_box(L), W.wall_images(L, frozen), sub=1)
+    _, _, srt, _ = O.clist_build(L, host(d)[:w.n_solvent])
+    if order == "shuffled":
+        srt = srt[np.random.default_rng(1).permutation(len(srt))]
+    if order == "one":
+        srt = srt[np.argmax(srt[:, 2])][None]
+    par = (25.0, 4.5, O.dpd_sigma(0.5, 4.5, 1e-3), 0.25)
+    ff = np.ones((len(srt), 3), np.float32)
+    want, npair = W.wall_forces(L, srt, ref, wpp, wst, par, np.float32(0.37), ff.copy())
+    fd = torch.as_tensor(ff).cuda()
+    w.force(U.PairDpd(*par), torch.as_tensor(np.ascontiguousarray(srt)).cuda(), fd, seed=np.float32(0.37))
+    assert w.pairs() == npair and npair > 0
+    assert np.array_equal(host(fd).view(np.uint32), want.view(np.uint32))
+    w.close()
+    q.close()
