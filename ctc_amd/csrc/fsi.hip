@@ -130,7 +130,7 @@ __global__ __launch_bounds__(64 * FI_WAVES) void k_fsi_instance(FsiK K, const in
                                                                 unsigned long long *pairs) {
     struct Wave {
         float4 hp[FI_HOMES], hv[FI_HOMES];   // position and noise index; velocity and seed
-        unsigned item[3][FI_CAP];            // a pair: home << 27 | solvent particle; then its force
+        unsigned item[3][FI_CAP];            // a pair: solvent particle, home; then its force
     };
     __shared__ Wave lds[FI_WAVES];
     __shared__ int count[FI_WAVES];
@@ -166,8 +166,9 @@ __global__ __launch_bounds__(64 * FI_WAVES) void k_fsi_instance(FsiK K, const in
     int sel = wave_any(m > 64) ? 0 : -1, skip = 0;
     for (;;) {
         const int nc = sel < 0 || sel == row ? m - skip : 0;
-        const unsigned byte = (unsigned)(nc > 0 ? j + skip : 0) * 16u;
-        const Mask64 mk = test64(nc, rx, ry, rz, [&](int k) { return pos_at(spos, byte, k); });
+        // (the bound solvent may exceed the 2^28 particles of 32-bit offsets)
+        const UDX_GLOBAL f4v *const cand = spos + (nc > 0 ? j + skip : 0);
+        const Mask64 mk = test64(nc, rx, ry, rz, [&](int k) { return pos_at(cand, 0u, k); });
         const int end = wave_scan_add(__popc(mk.w[0]) + __popc(mk.w[1]));
         const int off = end - (__popc(mk.w[0]) + __popc(mk.w[1]));
         const int T = __builtin_amdgcn_readlane(end, 63);
@@ -182,8 +183,10 @@ __global__ __launch_bounds__(64 * FI_WAVES) void k_fsi_instance(FsiK K, const in
                 unsigned b = mk.w[c];
                 while (wave_any(b != 0u)) {
                     const int k = __builtin_clz(b | 1u);
-                    if (b && at >= 0 && at < FI_CAP)
-                        S.item[0][at] = (unsigned)h << 27 | (unsigned)(j + skip + 32 * c + k);
+                    if (b && at >= 0 && at < FI_CAP) {
+                        S.item[0][at] = (unsigned)(j + skip + 32 * c + k);
+                        S.item[1][at] = (unsigned)h;
+                    }
                     at += b ? 1 : 0;
                     b &= ~(0x80000000u >> k);
                 }
@@ -192,9 +195,9 @@ __global__ __launch_bounds__(64 * FI_WAVES) void k_fsi_instance(FsiK K, const in
             const int Tw = min(T - c0, FI_CAP);
             auto in_of = [&](int q) {
                 // a lane past the list takes the first instance and solvent particle
-                const unsigned e = q < Tw ? S.item[0][q] : 0u, b = e & 0x7FFFFFFu;
-                const float4 hp = S.hp[e >> 27], hv = S.hv[e >> 27];
-                const f3v pb = pos_at(spos, b * 16u, 0), vb = pos_at(svel, b * 16u, 0);
+                const unsigned b = q < Tw ? S.item[0][q] : 0u, e = q < Tw ? S.item[1][q] : 0u;
+                const float4 hp = S.hp[e], hv = S.hv[e];
+                const f3v pb = pos_at(spos + b, 0u, 0), vb = pos_at(svel + b, 0u, 0);
                 const unsigned lid = (unsigned)__float_as_int(hp.w);
                 FsiIn o;
                 o.dx = hp.x - pb.x;

@@ -173,6 +173,38 @@ def test_vertex_side_bit_exact(ctx, rho, nv):
     f.close()
 
 
+@pytest.mark.parametrize("first", [(1 << 27) - 300, (1 << 28) - 300])
+def test_vertex_side_large_indices(ctx, first):
+    """solvent indices on both sides of 2^27 and of 2^28: the particles before
+    the first cell are in no cell (their positions, the box centre, are out of
+    every vertex's reach)"""
+    L = (8, 8, 8)
+    say("vertex side, first solvent particle", first)
+    starts, _, srt, _ = O.clist_build(L, particles(L, 5000, 8))
+    starts = (starts + first).astype(np.int32)
+    rng = np.random.default_rng(3)
+    opp = np.zeros((40, 6), np.float32)
+    opp[:, :3] = rng.uniform(2.1, 5, (40, 3)) * rng.choice([-1, 1], (40, 3))
+    par = (2.6666667, 8.0, O.dpd_sigma(0.0444, 8.0, 5e-4), 0.25)
+    seeds = np.array([0.31, 0.77], np.float32)
+    n = first + len(srt)
+    pp = np.zeros((n, 6), np.float32)   # pages that are never touched take no memory
+    pp[first:] = srt
+    fo, fs, npair = R.fsi_forces(L, pp, starts, opp, par, seeds)
+    del pp
+    pd = torch.zeros((n, 6), device="cuda")
+    pd[first:] = torch.as_tensor(srt).cuda()
+    fd, st, od = torch.zeros((n, 3), device="cuda"), torch.as_tensor(starts).cuda(), torch.zeros((40, 3), device="cuda")
+    f = U.Fsi(ctx, L, 40)
+    f.bind_solvent(pd, fd, U._ptr(st))
+    f.apply(U.PairDpd(*par), torch.as_tensor(opp).cuda(), od, seeds=seeds)
+    assert f.pairs() == npair and npair > 0
+    assert np.array_equal(host(od).view(np.uint32), fo.view(np.uint32))
+    assert np.array_equal(host(fd[first:]).view(np.uint32), fs[first:].view(np.uint32))
+    assert not bool(fd[:first].any())
+    f.close()
+
+
 @pytest.mark.parametrize("L,n", [((2, 3, 4), 257), ((6, 4, 8), 64), ((6, 4, 8), 1500), ((1, 5, 2), 65), ((16, 16, 16), 1)])
 def test_contact_bit_exact(ctx, L, n):
     """membrane contact: rows of cells with none, one and many points (four are
