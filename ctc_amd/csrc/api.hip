@@ -689,6 +689,7 @@ static int flu_step(udx_flu *f, const float *seeds_dev, const float *fsi_seeds, 
         f->wall->t = f->t;
         wv = wall_vel_view(f->wall->wvel, f->t);
         sdf = wall_sdf(f->wall);
+        d.fluid = wall_set(f->wall)->fluid;
     }
     // Without objects the gather also evaluates the wall forces and moves the
     // particles (into the other pair of streams, which the next step's reorder

@@ -1858,21 +1858,36 @@ double split_edges = 1048576.0;   // udx_dpd_set_split_edges
 bool split_halo(const DpdLaunch &a) { return a.eidx && a.periodic && edge_estimate(a.box, a.nmax) >= split_edges; }
 
 // One block per 64 particles (k_dpd_coop) while its blocks come to at most
-// twelve per CU.  A lane-per-particle launch is one latency chain long up to
-// about that size; past it the chip has waves enough to hide the chain, and the
-// barriers of the blocks cost more.  Measured, one step with its cell list
-// (lane per particle -> block): density 10, 138 thousand particles 191 -> 140
-// us, 220 thousand 207 -> 191, 328 thousand 228 -> 252; density 5, 240 thousand
-// 165 -> 166; density 3, 144 thousand 129 -> 120, 240 thousand 143 -> 156.
-// Without x slabs a run has twice the candidates, which the blocks test one
+// twelve per CU, fewer in dense boxes.  A lane-per-particle launch is one
+// latency chain long up to about that size; past it the chip has waves enough to
+// hide the chain, and the barriers of the blocks cost more.  Measured, one step
+// with its cell list (lane per particle -> block): density 10, 127 thousand
+// particles 140 -> 112 us, 197 thousand 156 -> 147; density 6, 197 thousand 124
+// -> 123; density 3, 160 thousand 96 -> 93, 197 thousand 103 -> 108.
+// Without x slabs a run has a third more candidates, which the blocks test one
 // row to a wave: level at 195 thousand (182 -> 185), so the line is lower.
-bool dpd_small(const DpdK &k, int nmax) { return ceil_div(nmax, 64) <= (k.bstarts ? 12 : 8) * 256; }
+// A block with more than 64 candidates in a run of any of its lanes takes the
+// runs one by one; with a mean of 36 in a run (density 16 with x slabs, 12
+// without) hardly any has, with 48 nearly all have, and then the blocks win
+// only while the chip runs them at once: density 16, 163 thousand particles 208
+// -> 198 us; density 18, 130 thousand 210 -> 186, 159 thousand 217 -> 270;
+// density 20, 63 thousand 223 -> 206, 98 thousand 224 -> 256; density 24, 32
+// thousand 251 -> 192, 66 thousand 257 -> 339; density 30, 33 thousand 303 ->
+// 280, 195 thousand 383 -> 990; density 45, 33 thousand 448 -> 355, 65 thousand 474 ->
+// 598; without slabs density 14, 96 thousand 183 ->
+// 153, 130 thousand 171 -> 212; density 18, 31 thousand 199 -> 171, 65 thousand
+// 208 -> 315.  (The blocks' offsets into the wall particles are 32 bits.)
+bool dpd_small(const DpdLaunch &a) {
+    const double run = a.nmax / (a.fluid * a.box.ncells()) * (a.bstarts ? 2.25 : 3.0);
+    const double top = a.bstarts ? 12.0 : 8.0, line = top - (top - 2.5) * fmin(fmax(run - 36.0, 0.0) / 12.0, 1.0);
+    return ceil_div(a.nmax, 64) <= (int)(line * 256.0) && (!a.move || a.move->nwall < (1 << 28));
+}
 
 template <int WR, bool EXACT>
-int launch_dpd(hipStream_t s, const DpdK &k, int nmax) {
+int launch_dpd(hipStream_t s, const DpdK &k, int nmax, bool small) {
     const dim3 g(ceil_div(nmax, DPD_THREADS)), b(DPD_THREADS);
     const Box box{{k.Lx, k.Ly, k.Lz}};
-    if (dpd_small(k, nmax) && !(k.eidx && k.periodic && edge_estimate(box, nmax) >= split_edges)) {
+    if (small && !(k.eidx && k.periodic && edge_estimate(box, nmax) >= split_edges)) {
         const dim3 gc(ceil_div(nmax, 64)), bc(CO_THREADS);
         if (k.opos && k.sdf.tex) hipLaunchKernelGGL((k_dpd_coop<WR, 2>), gc, bc, 0, s, k);
         else if (k.opos) hipLaunchKernelGGL((k_dpd_coop<WR, 1>), gc, bc, 0, s, k);
@@ -1969,11 +1984,12 @@ int dpd_forces_mode(hipStream_t s, const DpdLaunch &a, int mode) {
         UDX_CHECK(e == hipSuccess, UDX_EHIP, "dpd: stress kernel launch: %s", hipGetErrorString(e));
         return UDX_OK;
     }
+    const bool small = dpd_small(a);
     if (exact) {
-        if (sp == 0.25f) return launch_dpd<WR_QUARTER, true>(s, k, a.nmax);
-        if (sp == 0.5f) return launch_dpd<WR_HALF, true>(s, k, a.nmax);
-        if (sp == 1.0f) return launch_dpd<WR_ONE, true>(s, k, a.nmax);
-        return launch_dpd<WR_POW, true>(s, k, a.nmax);
+        if (sp == 0.25f) return launch_dpd<WR_QUARTER, true>(s, k, a.nmax, small);
+        if (sp == 0.5f) return launch_dpd<WR_HALF, true>(s, k, a.nmax, small);
+        if (sp == 1.0f) return launch_dpd<WR_ONE, true>(s, k, a.nmax, small);
+        return launch_dpd<WR_POW, true>(s, k, a.nmax, small);
     }
     if (mode == UDX_MODE_HALF) {
         UDX_CHECK(a.acc, UDX_EINVAL, "dpd: the half-shell mode needs FP64 accumulators");
@@ -1990,10 +2006,10 @@ int dpd_forces_mode(hipStream_t s, const DpdLaunch &a, int mode) {
         UDX_LAUNCHED();
         return UDX_OK;
     }
-    if (sp == 0.25f) return launch_dpd<WR_QUARTER, false>(s, k, a.nmax);
-    if (sp == 0.5f) return launch_dpd<WR_HALF, false>(s, k, a.nmax);
-    if (sp == 1.0f) return launch_dpd<WR_ONE, false>(s, k, a.nmax);
-    return launch_dpd<WR_POW, false>(s, k, a.nmax);
+    if (sp == 0.25f) return launch_dpd<WR_QUARTER, false>(s, k, a.nmax, small);
+    if (sp == 0.5f) return launch_dpd<WR_HALF, false>(s, k, a.nmax, small);
+    if (sp == 1.0f) return launch_dpd<WR_ONE, false>(s, k, a.nmax, small);
+    return launch_dpd<WR_POW, false>(s, k, a.nmax, small);
 }
 
 int dpd_forces(hipStream_t s, const DpdLaunch &a) { return dpd_forces_mode(s, a, 0); }

@@ -147,6 +147,7 @@ struct DpdLaunch {
     const FragTables *frag;
     Box box;
     int nmax;               // launch bound (>= particles)
+    float fluid = 1.f;      // share of the box that holds particles (about; walls fill the rest)
     int periodic;
     udx_pair_dpd par;
     const float *seeds;     // device, 27 floats
@@ -256,6 +257,7 @@ struct WallSet {
     float *pp_aos;   // the same in AoS (velocity 0)
     float *frozen;   // the frozen particles in freeze order (AoS), the restart template
     int n, nfrozen;  // all wall particles (frozen + periodic images), frozen ones
+    float fluid = 1.f;   // share of the particles that the freeze left in the solvent
 };
 void sdf_texture_size(const int L[3], int T[3]);
 int sdf_build(hipStream_t s, SdfField *q, const float ext[3], const int N[3], const float *D_host);

@@ -597,6 +597,7 @@ int wall_build(hipStream_t s, WallSet *w, const SdfField *q, int *n, float *pp) 
         return st;
     }
     *n = nb;
+    if (nb > 0) w->fluid = (float)nb / (float)n0;
     return wall_build_frozen(s, w, q, nw, frozen);
 }
 

@@ -84,6 +84,38 @@ def test_step_bit_exact(ctx, L, n, clump, spow):
     assert np.array_equal(got.view(np.uint32), ref.view(np.uint32))
 
 
+@pytest.mark.parametrize("L,rho", [((11, 12, 12), 24), ((12, 12, 12), 24), ((9, 8, 9), 63), ((9, 8, 9), 64),
+                                   ((23, 20, 20), 14), ((24, 20, 20), 18)])
+@pytest.mark.parametrize("slabs", [True, False])
+def test_dense_line_bit_exact(ctx, L, rho, slabs):
+    """dense boxes on both sides of the line between the block kernel and the
+    lane-per-particle kernel, which falls with the candidates of a run"""
+    n = rho * L[0] * L[1] * L[2]
+    say("dense line", L, rho, n, slabs)
+    pp, seeds = particles(L, n, 5), O.seeds_table(1)
+    par = (2.5, 4.5, O.dpd_sigma(0.05, 4.5, 5e-4), 0.25)
+    if slabs:
+        flu = U.Flu(ctx, L, n, U.PairDpd(*par), DT)
+        d = torch.as_tensor(pp).cuda()
+        flu.set_pp(d)
+        flu.run(1, seeds)
+        flu.get_pp(d)
+        got, npair = host(d), flu.pairs()
+        flu.close()
+        want, total = O.flu_step(L, pp, par, seeds[0], DT, nthreads=8)
+    else:
+        starts, counts, srt, _ = O.clist_build(L, pp)
+        want, total = O.dpd_forces(L, srt, starts, counts, par, seeds[0], nthreads=8)
+        f = U.FluForces(ctx, L, n)
+        sd, ff = torch.as_tensor(starts).cuda(), torch.zeros((n, 3), device="cuda")
+        f.prepare(torch.as_tensor(srt).cuda())
+        f.apply(U.PairDpd(*par), U._ptr(sd), ff, seeds=seeds[0])
+        got, npair, total = host(ff), f.pairs(), total // 2
+        f.close()
+    assert npair == total
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+
+
 @pytest.mark.parametrize("L,n,clump", CASES[1:])
 @pytest.mark.parametrize("periodic", [True, False])
 def test_whole_cells_bit_exact(ctx, L, n, clump, periodic):
