@@ -1756,12 +1756,37 @@ __global__ __launch_bounds__(1024) void k_frag_tables(const int *starts, int Lx,
     else frag_table<1024>(c.n, c, fss + off);
 }
 
+// The counts of a batch with x faces of more than FRAG_FACE_BATCH cells
+// (k_frag_counts for every box).  The launch costs the batch 5 to 9 us, and a
+// z face is a run of memory (one launch against two: 64 boxes of 8 to 48 cells
+// a side 10.5 us, 15.0; a z face of 96 x 96 cells 13.9, 15.4; an x face of 64 x
+// 64 11.2, 10.2, of 96 x 96 21, 14.6; a 96^3 box 31, 16).
+constexpr int FRAG_FACE_BATCH = 6144;
+__global__ __launch_bounds__(256) void k_frag_counts_batch(int nbox, const int *fbase, const int *foff, const int *coff,
+                                                           const int4 *boxL, const int *starts, int *cnt) {
+    const int g = blockIdx.x * 256 + threadIdx.x;
+    if (g >= fbase[nbox]) return;
+    int b = 0, hi = nbox;
+    while (hi - b > 1) {
+        const int mid = (b + hi) >> 1;
+        if (fbase[mid] <= g) b = mid;
+        else hi = mid;
+    }
+    const int *const off = foff + 27 * b, gl = g - fbase[b];
+    int f = 0;
+    while (f < 25 && gl >= off[f + 1]) f++;
+    const int4 L = boxL[b];
+    const FragCells c(starts + coff[b], L.x, L.y, L.z, f);
+    const int h = gl - off[f];
+    if (h < c.n) cnt[g] = c(h);
+}
+
 // the same for every box of a batch, 26 blocks a box; the first blocks also
 // copy the step's seeds of every box and clear the edge list counters (the
 // step counter advances later in the step)
 __global__ __launch_bounds__(256) void k_frag_tables_batch(int nbox, const int *fbase, const int *foff,
                                                            const int *coff, const int4 *boxL, const int *starts,
-                                                           int *fss, int *ecount, const float *table,
+                                                           const int *cnt, int *fss, int *ecount, const float *table,
                                                            const int *step, float *seeds) {
     const int g = blockIdx.x * 256 + threadIdx.x;
     if (g < 27 * nbox) seeds[g] = table[(long)*step * 27 * nbox + g];
@@ -1769,7 +1794,9 @@ __global__ __launch_bounds__(256) void k_frag_tables_batch(int nbox, const int *
     const int b = blockIdx.x / 26, f = blockIdx.x % 26;
     const int4 L = boxL[b];
     const FragCells c(starts + coff[b], L.x, L.y, L.z, f);
-    frag_table<256>(c.n, c, fss + fbase[b] + foff[27 * b + f]);
+    const int off = fbase[b] + foff[27 * b + f];
+    if (cnt) frag_table<256>(c.n, [&](int h) { return cnt[off + h]; }, fss + off);
+    else frag_table<256>(c.n, c, fss + off);
 }
 
 DpdK make_k(const DpdLaunch &a) {
@@ -1913,6 +1940,8 @@ int launch_dpd(hipStream_t s, const DpdK &k, int nmax, bool small) {
 
 }  // namespace
 
+bool frag_counted_batch(const Box &b) { return (long)b.L[1] * b.L[2] > FRAG_FACE_BATCH; }
+
 int frag_alloc(FragTables *t, const Box &b) {
     *t = FragTables{};
     int off = 0;
@@ -1950,9 +1979,15 @@ int frag_build(hipStream_t s, const FragTables *t, const Box &b, const int *star
 }
 
 int frag_build_batch(hipStream_t s, int nbox, const int *fbase, const int *foff, const int *coff, const int4 *boxL,
-                     const int *starts, int *fss, int *ecount, const float *table, const int *step, float *seeds) {
+                     const int *starts, int ftot, int *cnt, int *fss, int *ecount, const float *table, const int *step,
+                     float *seeds) {
+    if (cnt) {
+        hipLaunchKernelGGL(k_frag_counts_batch, dim3(ceil_div(ftot, 256)), dim3(256), 0, s, nbox, fbase, foff, coff,
+                           boxL, starts, cnt);
+        UDX_LAUNCHED();
+    }
     hipLaunchKernelGGL(k_frag_tables_batch, dim3(26 * nbox), dim3(256), 0, s, nbox, fbase, foff, coff, boxL, starts,
-                       fss, ecount, table, step, seeds);
+                       cnt, fss, ecount, table, step, seeds);
     UDX_LAUNCHED();
     return UDX_OK;
 }

@@ -141,7 +141,7 @@ struct udx_ens {
     int *ecount, *eidx;            // edge lists of the gather's halo pass (a counter per box)
     float4 *ef;
     ClistBufs cl;
-    int *fss;
+    int *fss, *fcnt;
     float *seeds_table, *seeds_cur, *seeds_host;
     int *step;
     unsigned long long *pairs;
@@ -218,7 +218,8 @@ static int ens_step(udx_ens *e, int cur, int *next) {
     const int a = cur, b = 1 - cur, n = e->ntot;
     if (!e->counted) UDX_TRY(ens_count(e, a));
     UDX_TRY(clist_finish_f4(s, &e->cl, n, e->pos[a], e->vel[a], e->pos[b], e->vel[b]));
-    UDX_TRY(frag_build_batch(s, e->nbox, e->fbase, e->foff, e->coff, e->boxL, e->cl.starts, e->fss, e->ecount,
+    UDX_TRY(frag_build_batch(s, e->nbox, e->fbase, e->foff, e->coff, e->boxL, e->cl.starts, e->ftot, e->fcnt,
+                             e->fss, e->ecount,
                              e->seeds_table, e->step, e->seeds_cur));
     UDX_TRY(dpd_forces_batch(s, e->batch[b], e->mode, e->variant));
     const bool fused = e->mode != UDX_MODE_HALF;
@@ -316,6 +317,7 @@ int udx_ens_fin(udx_ens *e) {
     dev_free(e->boxL);
     dev_free(e->mb);
     dev_free(e->fss);
+    dev_free(e->fcnt);
     dev_free(e->seeds_table);
     dev_free(e->seeds_cur);
     dev_free(e->step);
@@ -399,6 +401,9 @@ int udx_ens_ini(udx_ctx *ctx, int nbox, const udx_ens_box *boxes, udx_ens **out)
     if (!st) st = dev_alloc(&e->ef, (size_t)(e->ntot > 0 ? e->ntot : 1));
     if (!st) st = clist_alloc(&e->cl, Box{{e->ctot, 1, 1}}, e->ntot > 0 ? e->ntot : 1, SOLVENT_SUB);
     if (!st) st = dev_alloc(&e->fss, (size_t)e->ftot + 1);
+    bool counted = false;
+    for (int b = 0; b < nbox; b++) counted |= frag_counted_batch(Box{{boxes[b].L[0], boxes[b].L[1], boxes[b].L[2]}});
+    if (!st && counted) st = dev_alloc(&e->fcnt, (size_t)e->ftot);
     if (!st) st = dev_alloc(&e->seeds_cur, 27 * (size_t)nbox);
     if (!st) st = dev_alloc(&e->step, 1);
     if (!st) st = dev_alloc(&e->pairs, 1);

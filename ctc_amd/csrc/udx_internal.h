@@ -131,9 +131,12 @@ struct StepSeeds {
 int frag_build(hipStream_t s, const FragTables *t, const Box &b, const int *starts, int *ecount = nullptr,
                const StepSeeds &seeds = StepSeeds{});
 // the same for the boxes of a batch, laid end to end: fragment tables at
-// fbase + foff (27 per box), cells from coff; seeds of every box
+// fbase + foff (27 per box, ftot entries in all), cells from coff; cnt: ftot
+// counts where a box has an x face large enough, else null; seeds of every box
+bool frag_counted_batch(const Box &b);
 int frag_build_batch(hipStream_t s, int nbox, const int *fbase, const int *foff, const int *coff, const int4 *boxL,
-                     const int *starts, int *fss, int *ecount, const float *table, const int *step, float *seeds);
+                     const int *starts, int ftot, int *cnt, int *fss, int *ecount, const float *table, const int *step,
+                     float *seeds);
 
 // entries a gather may read past a lane's last candidate (values unused): the
 // position streams it reads have this many more than their particles

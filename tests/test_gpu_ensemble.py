@@ -138,6 +138,35 @@ def test_ensemble_exact_equals_oracle(ctx):
         assert np.array_equal(got[off[b]:off[b + 1]].view(np.uint32), ref.view(np.uint32)), "box %d" % b
 
 
+@pytest.mark.parametrize("graph,ys", [(False, 79), (True, 79), (False, 76)])
+def test_large_faces_equal_oracle(ctx, graph, ys):
+    """boxes with x faces above and below 6144 cells (above, the fragment
+    cells are counted in a launch of their own), other large faces, small boxes"""
+    nsteps = 4
+    boxes, pps = make_boxes(5, 11, edges=(3, 6))
+    for b, L in ((0, (67, 3, 65)), (2, (3, ys, 80)), (4, (66, 64, 3))):
+        rng = np.random.default_rng(b)
+        n = 2 * L[0] * L[1] * L[2] + 1
+        pp = np.zeros((n, 6), np.float32)
+        pp[:, :3] = inside(rng.uniform(-0.5, 0.5, (n, 3)) * np.array(L), L)
+        pp[:, 3:] = rng.normal(0, 0.5, (n, 3))
+        boxes[b] = dict(boxes[b], L=L, n=n)
+        pps[b] = pp
+    seeds = U.ens_trunk_seeds(5, nsteps)
+    say("ensemble, large faces", [b["L"] for b in boxes], graph)
+    got, pairs = run_ensemble(ctx, boxes, pps, nsteps, seeds, True, graph=graph)
+    off, total = 0, 0
+    for b, box in enumerate(boxes):
+        ref = pps[b]
+        for k in range(nsteps):
+            ref, p = O.flu_step(box["L"], ref, box["par"], seeds[k, b], box["dt"], accel=box["accel"], nthreads=8)
+            total += p
+        assert len(ref) == box["n"]
+        assert np.array_equal(got[off:off + box["n"]].view(np.uint32), ref.view(np.uint32)), "box %d" % b
+        off += box["n"]
+    assert pairs == total
+
+
 def test_graph_replays_match_eager(ctx):
     """The captured step pair, replayed with eager work and host syncs in
     between, gives the eager result after every replay."""
