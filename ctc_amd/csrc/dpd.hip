@@ -317,8 +317,10 @@ __device__ __forceinline__ void finish(const DpdK &A, const DpdP &P, bool mine, 
 // global memory.  Each lane sums its pairs in candidate order, bulk first.
 //
 // MOVE (one launch of a periodic box, float4 forces): 1 the particles are
-// also moved (FusedMove), 2 the same with walls.
-template <int WR, bool EXACT, int NT, int QC, int SC, bool STRESS = false, int PHASE = PH_ALL, int MOVE = 0>
+// also moved (FusedMove), 2 the same with walls.  OWN: the cell list is the
+// library's own, which leaves out particles without a finite position.
+template <int WR, bool EXACT, int NT, int QC, int SC, bool STRESS = false, int PHASE = PH_ALL, int MOVE = 0,
+          bool OWN = (MOVE != 0)>
 __device__ __forceinline__ void dpd_block(const DpdK &A, int first) {
     static_assert(QC >= 8 && (QC & (QC - 1)) == 0, "the queue length is a power of two");
     // 16-bit bulk entries, one region of QC * 128 bytes per wave, which the
@@ -429,6 +431,16 @@ __device__ __forceinline__ void dpd_block(const DpdK &A, int first) {
         add(pair_force(va, a, xa), a);
         add(pair_force(vb, b, xb), b);
         head += fl < 2u * STEP ? fl : 2u * STEP;
+    };
+    // a lane without pairs has added its idle slots' zeros only, which are no
+    // zeros where its position is not finite
+    auto no_pairs = [&]() {
+        if (OWN) return;
+        const bool none = npair == 0;
+        fx = none ? f0x : fx;
+        fy = none ? f0y : fy;
+        fz = none ? f0z : fz;
+        if (STRESS && none) sxx = sxy = sxz = syy = syz = szz = 0.f;
     };
     // room for `need` more entries in every lane (need <= 2 DRAIN_STEPS)
     auto make_room = [&](auto pass, unsigned need) {
@@ -598,6 +610,7 @@ __device__ __forceinline__ void dpd_block(const DpdK &A, int first) {
         if (!STRESS && QC >= 16) share_tail();
         drain(PassTag<true>{});
         npair = (int)(tail / STEP);   // every entry queued was a pair
+        if (PHASE == PH_BULK) no_pairs();
     }
 
     // ---- halo pass: the cells across the periodic boundary.  The noise
@@ -725,6 +738,7 @@ __device__ __forceinline__ void dpd_block(const DpdK &A, int first) {
         while (wave_any(ht != hh)) hstep();
         __builtin_amdgcn_wave_barrier();
     }
+    if (PHASE != PH_BULK) no_pairs();
 
     // ---- wall pass (MOVE == 2): the particles that are not sdf_far and the
     // frozen wall particles in the 27 cells of the wall cell list around
@@ -885,7 +899,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(batch_waves(
         else hi = mid;
     }
     const DpdK &A = boxes[lo];
-    dpd_block<WR, EXACT, NT, QC, SCAP_BATCH, false, PHASE>(A, A.i0 + (blk - bblock[lo]) * NT);
+    dpd_block<WR, EXACT, NT, QC, SCAP_BATCH, false, PHASE, 0, true>(A, A.i0 + (blk - bblock[lo]) * NT);
 }
 
 // ---------------------------------------------------------------- one block per 64 particles

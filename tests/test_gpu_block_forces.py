@@ -287,6 +287,36 @@ def test_not_a_number_hits_nothing(ctx, nan, c):
     assert np.array_equal(out[0][0].view(np.uint32), out[1][0].view(np.uint32))
 
 
+@pytest.mark.parametrize("L,split", [((8, 6, 8), False), ((26, 26, 26), False), ((26, 26, 26), True)])
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+def test_no_position_no_force(ctx, L, split, bad):
+    """a particle whose position is not finite has no pairs: nothing is added
+    to its own force (the block kernel, the lane-per-particle kernel and its
+    split passes), and its stress stays"""
+    rho, k = 8, 1500
+    n = rho * L[0] * L[1] * L[2]
+    say("no position", L, split, bad)
+    starts, _, srt, _ = O.clist_build(L, particles(L, n, 4))
+    srt[k, 1] = bad
+    par, seeds = U.PairDpd(25.0, 4.5, O.dpd_sigma(0.5, 4.5, 1e-3), 0.25), O.seeds_table(1)[0]
+    f = U.FluForces(ctx, L, n)
+    pd, sd = torch.as_tensor(srt).cuda(), torch.as_tensor(starts).cuda()
+    f.prepare(pd)
+    try:
+        if split:
+            U.set_split_edges(0.0)
+        ff = torch.ones((n, 3), device="cuda")
+        f.apply(par, U._ptr(sd), ff, seeds=seeds)
+    finally:
+        U.set_split_edges(1048576.0)
+    assert host(ff[k]).tolist() == [1.0, 1.0, 1.0]
+    assert bool(torch.isfinite(ff).all())
+    ff, ss = torch.ones((n, 3), device="cuda"), torch.ones((n, 6), device="cuda")
+    f.apply_stress(par, U._ptr(sd), ff, ss, seeds=seeds)
+    assert host(ff[k]).tolist() == [1.0] * 3 and host(ss[k]).tolist() == [1.0] * 6
+    f.close()
+
+
 @pytest.mark.parametrize("rho,order", [(3, "cells"), (30, "cells"), (30, "shuffled"), (45, "cells"), (45, "one")])
 def test_wall_rows_bit_exact(ctx, rho, order):
     """wall forces by a launch of their own: rows that a wave stages and rows
