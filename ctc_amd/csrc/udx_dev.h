@@ -26,11 +26,13 @@ __device__ constexpr float R_SQRT2  = 1.41421356237309514547f;
 // states are written out: the hardware orders a mode write against the vector
 // instructions before and after it (the compiler brackets its own division
 // sequences with mode writes the same way), and two writes of the register
-// need two instructions between them: the fma, and the squares of two chains
-// (one chain has a single square, hence its s_nop).  The chain bounds the
-// latency of every pair: with four s_nop 1 per round a lone wave took 775
-// cycles for two pairs of chains, 472 without (192 and 177 with five waves
-// per SIMD).
+// need two instructions between them: the fma inside a round, and between the
+// rounds of a chain the squares of its two values (a single value has one
+// square, hence its s_nop).  Nothing ties the squares of a chain's first round to
+// the place after the chain before, so each chain starts with the two wait
+// states (mode_gap).  The chain bounds the latency of every pair: with four
+// s_nop 1 per round a lone wave took 775 cycles for two pairs of chains, 472
+// without (192 and 177 with five waves per SIMD).
 __device__ __forceinline__ float t4_round_rz(float x2, float c8, float cm8) {
     float t, r;
     asm volatile(
@@ -61,9 +63,12 @@ __device__ __forceinline__ void t4_round_rz2(float a2, float b2, float c8, float
     *rb = ob;
 }
 
+__device__ __forceinline__ void mode_gap() { asm volatile("s_nop 1"); }
+
 // nine rounds (N = 18), the square rounded to nearest
 __device__ __forceinline__ float logistic18(float x) {
     const float c8 = 8.0f, cm8 = -8.0f;
+    mode_gap();
 #pragma unroll
     for (int k = 0; k < 9; k++) {
         float x2 = x * x;
@@ -75,6 +80,7 @@ __device__ __forceinline__ float logistic18(float x) {
 __device__ __forceinline__ void logistic18x2(float *xa, float *xb) {
     const float c8 = 8.0f, cm8 = -8.0f;
     float a = *xa, b = *xb;
+    mode_gap();
 #pragma unroll
     for (int k = 0; k < 9; k++) {
         float a2 = a * a, b2 = b * b;
