@@ -119,8 +119,8 @@ def test_dense_line_bit_exact(ctx, L, rho, slabs):
 @pytest.mark.parametrize("L,n,clump", CASES[1:])
 @pytest.mark.parametrize("periodic", [True, False])
 def test_whole_cells_bit_exact(ctx, L, n, clump, periodic):
-    """the module binding: no slab starts, forces added to AoS; also equal to
-    the lane-per-particle kernels (split halo forced)"""
+    """the module binding: no slab starts, forces added to AoS; periodic boxes
+    also with the lane-per-particle kernels (split halo forced)"""
     say("block forces, whole cells", L, n, clump, periodic)
     starts, counts, srt, _ = O.clist_build(L, particles(L, n, 4, clump))
     par = (25.0, 4.5, O.dpd_sigma(0.5, 4.5, 1e-3), 0.25)
@@ -130,7 +130,7 @@ def test_whole_cells_bit_exact(ctx, L, n, clump, periodic):
     f = U.FluForces(ctx, L, n)
     sd, pd = torch.as_tensor(starts).cuda(), torch.as_tensor(srt).cuda()
     try:
-        for edges in (1 << 20, 0):
+        for edges in (1 << 20, 0) if periodic else (1 << 20,):
             U.set_split_edges(edges)
             f.prepare(pd)
             ff = torch.as_tensor(f0).cuda()

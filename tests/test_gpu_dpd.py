@@ -191,8 +191,10 @@ def test_forces_fast_mode_tolerance(ctx, case):
 @pytest.mark.parametrize("case", CASES)
 def test_forces_split_halo_pass_same_bits(ctx, case):
     """The halo pass as a launch of its own over the listed boundary
-    particles (forced here for small boxes) gives the bits of the pass inside
-    the force kernel, in both modes, and the oracle's."""
+    particles (forced here for small boxes) gives the oracle's bits in both
+    modes, as does the launch these boxes take by themselves (a block per 64
+    particles; the halo pass inside the lane-per-particle kernel is compared
+    in test_gpu_lane_forces.py)."""
     L, rho, a, g, kBT, dt, spow = case
     pp = random_box(L, rho, 9)
     starts, counts, srt, _ = O.clist_build(L, pp)
