@@ -170,9 +170,12 @@ __device__ __forceinline__ void clist_count_one(bool valid, int i, float3 r, int
 // ---------------------------------------------------------------- DPD pair
 // Correctly rounded square root of a positive normal float: the product of
 // x and the hardware reciprocal root, corrected by its fma residual times half
-// that root.  Equal to the IEEE root for every float of [2^-24, 1] (checked
-// exhaustively on gfx950; the library's self-check entry point repeats the
-// check).  One transcendental, two products and two fma, 19 issue cycles of a
+// that root (one Newton step as in P. Markstein, "Computation of elementary
+// functions on the IBM RISC System/6000 processor", 1990).  Equal to the IEEE
+// root for every float of [2^-24, 1] with gfx950's estimates (checked
+// exhaustively there; the library's self-check entry point repeats the check);
+// a few dozen floats of the range would differ with an estimate off by one more
+// float.  One transcendental, two products and two fma, 19 issue cycles of a
 // wave; the hardware root moved to a neighbour by two residuals, compares and
 // selects took 37.  x = 0 gives NaN.
 __device__ __forceinline__ float sqrt_rn(float x) {

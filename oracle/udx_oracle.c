@@ -807,14 +807,16 @@ long orc_flu_step(const int L[3], int n, float *pp, float *scratch_pp, int *star
 static float f_bits(uint32_t u) { float f; memcpy(&f, &u, 4); return f; }
 static uint32_t bits_f(float f) { uint32_t u; memcpy(&u, &f, 4); return u; }
 
-static float dev_sqrt_fix(float x, float s) {
-    const float sd = f_bits(bits_f(s) - 1u), su = f_bits(bits_f(s) + 1u);
-    const float rd = fmaf(-sd, s, x), ru = fmaf(-su, s, x);
-    const float t = rd <= 0.f ? sd : s;
-    return ru > 0.f ? su : t;
+/* x y corrected by its residual times y / 2, y an estimate of 1 / sqrt(x)
+ * (Newton's step for the square root) */
+static float dev_sqrt(float x, float y) {
+    const float s = x * y;
+    return fmaf(fmaf(-s, s, x), 0.5f * y, s);
 }
 
-long orc_verify_sqrt_rn(float lo, float hi, int nthreads, int correct) {
+/* floats x of [lo, hi] whose root from the estimate `ulp` floats away from
+ * the one nearest to 1 / sqrt(x) differs from sqrtf; corrected = 0: x y alone */
+long orc_verify_sqrt_rn(float lo, float hi, int nthreads, int ulp, int corrected) {
     const uint32_t a = bits_f(lo), b = bits_f(hi);
     long bad = 0;
     (void)nthreads;
@@ -823,11 +825,9 @@ long orc_verify_sqrt_rn(float lo, float hi, int nthreads, int correct) {
     #pragma omp parallel for schedule(static, 1 << 16) reduction(+:bad) num_threads(nthreads)
 #endif
     for (long u = a; u <= (long)b; u++) {
-        const float x = f_bits((uint32_t)u), want = sqrtf(x);
-        for (int d = -1; d <= 1; d++) {
-            const float s = f_bits(bits_f(want) + (uint32_t)d);
-            if ((correct ? dev_sqrt_fix(x, s) : s) != want) bad++;
-        }
+        const float x = f_bits((uint32_t)u);
+        const float y = f_bits(bits_f((float)(1.0 / sqrt((double)x))) + (uint32_t)ulp);
+        if ((corrected ? dev_sqrt(x, y) : x * y) != sqrtf(x)) bad++;
     }
     return bad;
 }

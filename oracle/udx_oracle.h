@@ -290,17 +290,13 @@ int   orc_cnt_images(const int L[3], int n, const float *pp, float *img, int *im
 long  orc_cnt_forces(const int L[3], int n, const float *pp, orc_dpd_lj p, float seed_bulk, float seed_halo,
                      float *ff);
 
-/* ---- correctly rounded square root from the 1-ulp hardware root --------
- * The GPU kernels take the hardware square root s (within 1 ulp of the
- * exact value) and correct it with two fma residuals:
- *   s- = s - 1 ulp, s+ = s + 1 ulp;
- *   t = (x - s- s <= 0) ? s- : s;  result = (x - s+ s > 0) ? s+ : t
- * This checks every float x in [lo, hi] with every value the hardware may
- * give (the correctly rounded root and its two neighbours) against the
- * host's correctly rounded sqrtf.  Returns the number of failures.
- * correct = 0 checks the uncorrected hardware values instead (a control:
- * two failures per float). */
-long orc_verify_sqrt_rn(float lo, float hi, int nthreads, int correct);
+/* Exhaustive check of the formula of the GPU pair force's square root: from an
+ * estimate y of 1 / sqrt(x), s = x y and the result s + (x - s s) y / 2 with
+ * both sums fused.  For every float x in [lo, hi] the estimate is the float
+ * nearest to 1 / sqrt(x) moved by `ulp` floats.  Returns the number of results
+ * that differ from the host's correctly rounded sqrtf; corrected = 0 takes
+ * x y alone (a control). */
+long orc_verify_sqrt_rn(float lo, float hi, int nthreads, int ulp, int corrected);
 
 #ifdef __cplusplus
 }
