@@ -1899,14 +1899,19 @@ double split_edges = 1048576.0;   // udx_dpd_set_split_edges
 bool split_halo(const DpdLaunch &a) { return a.eidx && a.periodic && edge_estimate(a.box, a.nmax) >= split_edges; }
 
 // One block per 64 particles (k_dpd_coop) while its blocks come to at most
-// twelve per CU, fewer in dense boxes.  A lane-per-particle launch is one
-// latency chain long up to about that size; past it the chip has waves enough to
-// hide the chain, and the barriers of the blocks cost more.  Measured, one step
-// with its cell list (lane per particle -> block): density 10, 127 thousand
-// particles 140 -> 112 us, 197 thousand 156 -> 147; density 6, 197 thousand 124
-// -> 123; density 3, 160 thousand 96 -> 93, 197 thousand 103 -> 108.
+// twelve per CU, fewer in sparse and in dense boxes.  A lane-per-particle launch
+// is one latency chain long up to about that size; past it the chip has waves
+// enough to hide the chain, and the barriers of the blocks cost more.  Measured,
+// one step with its cell list (lane per particle -> block): density 10, 127
+// thousand particles 140 -> 112 us, 197 thousand 156 -> 147; density 6, 197
+// thousand 124 -> 123.
 // Without x slabs a run has a third more candidates, which the blocks test one
 // row to a wave: level at 195 thousand (182 -> 185), so the line is lower.
+// A sparse box's chain is short and its blocks have little to share: density 3,
+// 160 thousand 95 -> 91, 197 thousand 100 -> 106; density 1, 113 thousand 75 ->
+// 74, 160 thousand 79 -> 90; density 1/4, 64 thousand 66 -> 60, 129 thousand 83
+// -> 89; without slabs density 2, 113 thousand 69 -> 68, density 1/2, 64 thousand
+// 56 -> 51, 96 thousand 57 -> 61.
 // A block with more than 64 candidates in a run of any of its lanes takes the
 // runs one by one; with a mean of 36 in a run (density 16 with x slabs, 12
 // without) hardly any has, with 48 nearly all have, and then the blocks win
@@ -1914,14 +1919,16 @@ bool split_halo(const DpdLaunch &a) { return a.eidx && a.periodic && edge_estima
 // -> 198 us; density 18, 130 thousand 210 -> 186, 159 thousand 217 -> 270;
 // density 20, 63 thousand 223 -> 206, 98 thousand 224 -> 256; density 24, 32
 // thousand 251 -> 192, 66 thousand 257 -> 339; density 30, 33 thousand 303 ->
-// 280, 195 thousand 383 -> 990; density 45, 33 thousand 448 -> 355, 65 thousand 474 ->
-// 598; without slabs density 14, 96 thousand 183 ->
-// 153, 130 thousand 171 -> 212; density 18, 31 thousand 199 -> 171, 65 thousand
-// 208 -> 315.  (The blocks' offsets into the wall particles are 32 bits.)
+// 280, 195 thousand 383 -> 990; density 45, 33 thousand 448 -> 355, 65 thousand
+// 474 -> 598; without slabs density 14, 96 thousand 183 -> 153, 130 thousand 171
+// -> 212; density 18, 31 thousand 199 -> 171, 65 thousand 208 -> 315.  (The
+// blocks' offsets into the wall particles are 32 bits.)
 bool dpd_small(const DpdLaunch &a) {
+    // mean candidates of a run
     const double run = a.nmax / (a.fluid * a.box.ncells()) * (a.bstarts ? 2.25 : 3.0);
-    const double top = a.bstarts ? 12.0 : 8.0, line = top - (top - 2.5) * fmin(fmax(run - 36.0, 0.0) / 12.0, 1.0);
-    return ceil_div(a.nmax, 64) <= (int)(line * 256.0) && (!a.move || a.move->nwall < (1 << 28));
+    const double top = a.bstarts ? 12.0 : 8.0, sparse = top * fmin(0.46 + 0.06 * run, 1.0),
+                 dense = top - (top - 2.5) * fmin(fmax(run - 36.0, 0.0) / 12.0, 1.0);
+    return ceil_div(a.nmax, 64) <= (int)(fmin(sparse, dense) * 256.0) && (!a.move || a.move->nwall < (1 << 28));
 }
 
 template <int WR, bool EXACT>

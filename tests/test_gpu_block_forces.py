@@ -85,13 +85,14 @@ def test_step_bit_exact(ctx, L, n, clump, spow):
 
 
 @pytest.mark.parametrize("L,rho", [((11, 12, 12), 24), ((12, 12, 12), 24), ((9, 8, 9), 63), ((9, 8, 9), 64),
-                                   ((23, 20, 20), 14), ((24, 20, 20), 18)])
+                                   ((23, 20, 20), 14), ((24, 20, 20), 18), ((60, 41, 40), 1)])
 @pytest.mark.parametrize("slabs", [True, False])
-def test_dense_line_bit_exact(ctx, L, rho, slabs):
-    """dense boxes on both sides of the line between the block kernel and the
-    lane-per-particle kernel, which falls with the candidates of a run"""
+def test_line_bit_exact(ctx, L, rho, slabs):
+    """boxes on both sides of the line between the block kernel and the
+    lane-per-particle kernel, which falls with the candidates of a run in dense
+    boxes and with their lack in sparse ones"""
     n = rho * L[0] * L[1] * L[2]
-    say("dense line", L, rho, n, slabs)
+    say("line", L, rho, n, slabs)
     pp, seeds = particles(L, n, 5), O.seeds_table(1)
     par = (2.5, 4.5, O.dpd_sigma(0.05, 4.5, 5e-4), 0.25)
     if slabs:

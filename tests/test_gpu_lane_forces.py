@@ -1,7 +1,8 @@
 """The lane-per-particle force kernel, bit for bit against the CPU oracle, in
 boxes above the line up to which a block takes 64 particles: more than 196608
-particles with x slabs, more than 131072 without, or more than 40960 where a
-run of three cells holds 48 candidates or more.  Forces alone (periodic, not
+particles with x slabs, more than 131072 without, about half of that in sparse
+boxes, or more than 40960 where a run of three cells holds 48 candidates or
+more.  Forces alone (periodic, not
 periodic, the halo pass inside and as a launch of its own), the step that
 moves the particles (eager and captured) and the step with walls."""
 import sys
@@ -54,6 +55,7 @@ def particles(L, n, seed):
 
 # box, particles, spow
 BOXES = [((52, 51, 50), 132600, 0.5),       # density 1
+         ((70, 63, 65), 71663, 0.25),       # density 1/4, just above the line of sparse boxes
          ((7, 5, 1301), 136605 + 1, 1.0),   # thin and long, a last block with one particle
          ((3, 40, 139), 133440, 0.25),      # three cells across: every pair wraps along x or nearly so
          ((12, 11, 13), 41184, 0.25),       # density 24: runs staged in several chunks
