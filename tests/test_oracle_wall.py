@@ -81,6 +81,27 @@ def channel(L=(16, 12, 24), h=8.0, rho=4, seed=1):
     return s, pp
 
 
+def test_thin_box_closed_form():
+    """Box sides below the wall margin (6): the margin spans several periods of
+    the field.  The cubic B-spline of N samples of a cosine of one period is
+    the cosine times (2 + cos(2 pi / N)) / 3, up to the difference between the
+    spline and the cosine, below h^2 k^2 / 6 at the sample distance h; the
+    texture's linear interpolation adds at most H^2 k^2 / 8 per axis at the
+    texel distance H (k the wave number)."""
+    L, N = (4, 2, 4), (32, 32, 8)
+    x, y = (np.arange(N[0]) + 0.5) * L[0] / N[0], (np.arange(N[1]) + 0.5) * L[1] / N[1]
+    kx, ky = 2 * np.pi / L[0], 2 * np.pi / L[1]
+    D = np.broadcast_to(np.cos(kx * x)[None, None, :] + np.sin(ky * y)[None, :, None], N[::-1])
+    s = W.Sdf(L, np.array(L, np.float32), N, np.ascontiguousarray(D, np.float32).ravel())
+    r = np.random.default_rng(12).uniform(-1, 1, (4000, 3)) * (np.array(L) / 2 + 5.8)
+    ax, ay = ((2 + np.cos(2 * np.pi / n)) / 3 for n in N[:2])
+    want = ax * np.cos(kx * (r[:, 0] + L[0] / 2)) + ay * np.sin(ky * (r[:, 1] + L[1] / 2))
+    h = [L[c] / N[c] for c in range(2)] + [(L[c] + 12) / s.T[c] for c in range(2)]
+    tol = sum((h[c] * k) ** 2 / 6 + (h[2 + c] * k) ** 2 / 8 for c, k in enumerate((kx, ky)))
+    assert tol < 0.02
+    assert np.abs(s.eval(r) - want).max() < tol
+
+
 def test_freeze_labels_and_order():
     s, pp = channel()
     keep, wall = s.freeze(pp)
