@@ -11,7 +11,7 @@
 //
 // Here both sides gather, so no atomics are needed and the sums have a
 // fixed order:
-//  - k_fsi_instance: one thread per instance (vertex or image) in cell
+//  - k_fsi_instance: nine threads per instance (vertex or image) in cell
 //    order, one sum over its block; k_fsi_vertex_sum adds to each vertex
 //    its own sum, then its images' in halo-list order;
 //  - k_fsi_solvent: one thread per solvent particle over the vertex/image

@@ -309,7 +309,8 @@ __device__ __forceinline__ UDX_GLOBAL T *gptr(T *p) {
 }
 
 // x, y, z of the entry at a byte offset, plus K entries folded into the load.
-// The 32-bit offset (indices stay below 2^27) goes into the load beside the
+// The 32-bit offset (indices stay below 2^28: the callers' limits; else the index
+// goes into the base, a 64-bit sum) goes into the load beside the
 // base; a signed index takes five more instructions per particle to widen.
 __device__ __forceinline__ f3v pos_at(const UDX_GLOBAL f4v *p, unsigned byte, int k) {
     return *(const UDX_GLOBAL f3v *)((const UDX_GLOBAL char *)p + (size_t)byte + 16 * k);
